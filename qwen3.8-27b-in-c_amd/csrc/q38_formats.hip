@@ -29,309 +29,12 @@
  * pattern x86 gives, 0xffc00000).
  */
 #include "q38_device.h"
+#include "q38_format_decode.h"
 #include "q38_kernels.h"
-#include "q38_iq_grids.inc"
 
 namespace q38 {
 
 namespace {
-
-/* ---- codebooks, expanded at compile time --------------------------------- */
-
-#define Q38_IQ2_LEVEL(i) ((i) == 0 ? 8u : (i) == 1 ? 25u : 43u)
-#define Q38_IQ2_BYTE(c, k) Q38_IQ2_LEVEL(((c) >> (2 * (k))) & 3)
-#define Q38_IQ2_HALF(c, h) \
-    (Q38_IQ2_BYTE(c, 4 * (h)) | Q38_IQ2_BYTE(c, 4 * (h) + 1) << 8 | Q38_IQ2_BYTE(c, 4 * (h) + 2) << 16 | \
-     Q38_IQ2_BYTE(c, 4 * (h) + 3) << 24)
-#define Q38_IQ2_ENTRY(c) Q38_IQ2_HALF(c, 0), Q38_IQ2_HALF(c, 1),
-#define Q38_IQ3XXS_LEVEL(i) ((i) == 7 ? 62u : 8u * (i) + 4u)
-#define Q38_IQ3XXS_ENTRY(c) \
-    (Q38_IQ3XXS_LEVEL((c) & 7) | Q38_IQ3XXS_LEVEL(((c) >> 3) & 7) << 8 | Q38_IQ3XXS_LEVEL(((c) >> 6) & 7) << 16 | \
-     Q38_IQ3XXS_LEVEL(((c) >> 9) & 7) << 24),
-#define Q38_IQ3S_LEVEL(i) (2u * (i) + 1u)
-#define Q38_IQ3S_ENTRY(c) \
-    (Q38_IQ3S_LEVEL((c) & 7) | Q38_IQ3S_LEVEL(((c) >> 3) & 7) << 8 | Q38_IQ3S_LEVEL(((c) >> 6) & 7) << 16 | \
-     Q38_IQ3S_LEVEL(((c) >> 9) & 7) << 24),
-
-/* IQ2 grids: entry e, elements 4h..4h+3 at [2e + h]; IQ3 grids: entry e at [e] */
-__device__ const uint32_t g_iq2xxs[512] = {Q38_IQ2XXS_CODES(Q38_IQ2_ENTRY)};
-__device__ const uint32_t g_iq2xs[1024] = {Q38_IQ2XS_CODES(Q38_IQ2_ENTRY)};
-__device__ const uint32_t g_iq2s[2048] = {Q38_IQ2S_CODES(Q38_IQ2_ENTRY)};
-__device__ const uint32_t g_iq3xxs[256] = {Q38_IQ3XXS_CODES(Q38_IQ3XXS_ENTRY)};
-__device__ const uint32_t g_iq3s[512] = {Q38_IQ3S_CODES(Q38_IQ3S_ENTRY)};
-
-constexpr int8_t kIq4nl[16] = {Q38_IQ4NL_VALUES};
-constexpr uint32_t pack4(int a, int b, int c, int d)
-{
-    return (uint32_t)(uint8_t)a | (uint32_t)(uint8_t)b << 8 | (uint32_t)(uint8_t)c << 16 | (uint32_t)(uint8_t)d << 24;
-}
-constexpr uint32_t kIq4nlT0 = pack4(kIq4nl[0], kIq4nl[1], kIq4nl[2], kIq4nl[3]);
-constexpr uint32_t kIq4nlT1 = pack4(kIq4nl[4], kIq4nl[5], kIq4nl[6], kIq4nl[7]);
-constexpr uint32_t kIq4nlT2 = pack4(kIq4nl[8], kIq4nl[9], kIq4nl[10], kIq4nl[11]);
-constexpr uint32_t kIq4nlT3 = pack4(kIq4nl[12], kIq4nl[13], kIq4nl[14], kIq4nl[15]);
-
-/* GGML type ids (include/qwen38/qwen38_gguf.h:29-52) */
-enum : int {
-    kF32 = 0, kF16 = 1, kQ4_0 = 2, kQ4_1 = 3, kQ5_0 = 6, kQ5_1 = 7, kQ8_0 = 8, kQ2K = 10, kQ3K = 11, kQ5K = 13,
-    kIQ2XXS = 16, kIQ2XS = 17, kIQ3XXS = 18, kIQ1S = 19, kIQ4NL = 20, kIQ3S = 21, kIQ2S = 22, kIQ4XS = 23,
-    kBF16 = 30
-};
-
-__device__ __forceinline__ uint32_t ld16(const uint8_t *p)
-{
-    return (uint32_t)p[0] | (uint32_t)p[1] << 8;
-}
-/* 4 bytes at a 2-byte aligned address */
-__device__ __forceinline__ uint32_t ld32u(const uint8_t *p)
-{
-    const uint16_t *h = reinterpret_cast<const uint16_t *>(p);
-    return (uint32_t)h[0] | (uint32_t)h[1] << 16;
-}
-__device__ __forceinline__ uint32_t ld32a(const uint8_t *p) { return *reinterpret_cast<const uint32_t *>(p); }
-
-/* bytes of 0xff where bit k of `bits` (k < 4) is set */
-__device__ __forceinline__ uint32_t byte_mask4(uint32_t bits)
-{
-    return ((bits & 15u) * 0x00204081u & 0x01010101u) * 0xffu;
-}
-
-/* negate the bytes selected by mask (values 1..127, so no byte borrows) */
-__device__ __forceinline__ uint32_t negate_bytes(uint32_t v, uint32_t mask)
-{
-    return (v ^ mask) + (mask & 0x01010101u);
-}
-
-/* IQ2/IQ3 sign byte of a 7-bit index: even parity in bit 7 (ksigns_iq2xs) */
-__device__ __forceinline__ uint32_t sign_byte(uint32_t index)
-{
-    index &= 127u;
-    return index | (uint32_t)(__popc(index) & 1) << 7;
-}
-
-/* nibbles (one per byte) through the IQ4_NL table */
-__device__ __forceinline__ uint32_t iq4nl_bytes(uint32_t nib)
-{
-    const uint32_t sel = nib & 0x07070707u;
-    const uint32_t lo = __builtin_amdgcn_perm(kIq4nlT1, kIq4nlT0, sel);
-    const uint32_t hi = __builtin_amdgcn_perm(kIq4nlT3, kIq4nlT2, sel);
-    const uint32_t high = ((nib >> 3) & 0x01010101u) * 0xffu;
-    return (hi & high) | (lo & ~high);
-}
-
-__device__ __forceinline__ void k4_scale_min(int i, const uint8_t *p, int &sc, int &m)
-{
-    if (i < 4) {
-        sc = p[i] & 63;
-        m = p[i + 4] & 63;
-    } else {
-        sc = (p[i + 4] & 15) | ((p[i - 4] >> 6) << 4);
-        m = (p[i + 4] >> 4) | ((p[i] >> 6) << 4);
-    }
-}
-
-/* ---- Q8_K path: one lane's share of a super-block ------------------------- */
-
-/* The lane's packed weights q[g] (elements 32g + 4l .. +3) and integer
- * scales s[g] of the eight groups, the block's scale factor before the
- * activation scale, and (Q2_K, Q5_K: dmin; IQ1_S: unused) the second
- * factor.  IQ4_NL keeps its eight group scales in gd[]. */
-struct LaneBlock {
-    uint32_t q[8];
-    int s[8];
-    float d, dmin;
-    float gd[8];
-};
-
-template <int T>
-__device__ __forceinline__ uint32_t block_bytes()
-{
-    switch (T) {
-    case kQ2K: return 84;
-    case kQ3K: return 110;
-    case kQ5K: return 176;
-    case kIQ2XXS: return 66;
-    case kIQ2XS: return 74;
-    case kIQ2S: return 82;
-    case kIQ3XXS: return 98;
-    case kIQ3S: return 110;
-    case kIQ4XS: return 136;
-    case kIQ4NL: return 144;
-    default: return 50;   /* IQ1_S */
-    }
-}
-
-template <int T>
-__device__ __forceinline__ void decode_lane(const uint8_t *blk, int l, const uint32_t *iq1s_grid, LaneBlock &b)
-{
-    const int hi = l >= 4;
-    if constexpr (T == kQ2K) {
-        /* qwen38_quant.c:510-585 */
-        const uint32_t d0 = ld32a(blk + 16 + 4 * l), d1 = ld32a(blk + 48 + 4 * l);
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            b.q[g] = ((g < 4 ? d0 : d1) >> (2 * (g & 3))) & 0x03030303u;
-            b.s[g] = blk[2 * g + hi] & 15;
-        }
-        b.d = f16_to_f32(ld16(blk + 80));
-        b.dmin = f16_to_f32(ld16(blk + 82));
-    } else if constexpr (T == kQ3K) {
-        /* :587-662; scales :319-329 */
-        const uint32_t hm = ld32u(blk + 4 * l);
-        const uint32_t d0 = ld32u(blk + 32 + 4 * l), d1 = ld32u(blk + 64 + 4 * l);
-        const uint8_t *sc = blk + 96;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t low = ((g < 4 ? d0 : d1) >> (2 * (g & 3))) & 0x03030303u;
-            const uint32_t absent = ~(hm >> g) & 0x01010101u;
-            b.q[g] = low + absent * 0xfcu;   /* minus 4 where the high bit is clear */
-            const int i = 2 * g + hi;
-            const int lo4 = i < 8 ? sc[i] & 15 : sc[i - 8] >> 4;
-            const int hi2 = (sc[8 + i % 4] >> (2 * (i / 4))) & 3;
-            b.s[g] = (lo4 | hi2 << 4) - 32;
-        }
-        b.d = f16_to_f32(ld16(blk + 108));
-    } else if constexpr (T == kQ5K) {
-        /* :1636-1725 */
-        const uint32_t qh = ld32a(blk + 16 + 4 * l);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const uint32_t qs = ld32a(blk + 48 + 32 * c + 4 * l);
-            b.q[2 * c] = (qs & 0x0f0f0f0fu) + (((qh >> (2 * c)) & 0x01010101u) << 4);
-            b.q[2 * c + 1] = ((qs >> 4) & 0x0f0f0f0fu) + (((qh >> (2 * c + 1)) & 0x01010101u) << 4);
-            int sc0, m0, sc1, m1;
-            k4_scale_min(2 * c, blk + 4, sc0, m0);
-            k4_scale_min(2 * c + 1, blk + 4, sc1, m1);
-            b.s[2 * c] = sc0;
-            b.s[2 * c + 1] = sc1;
-        }
-        b.d = f16_to_f32(ld16(blk));
-        b.dmin = f16_to_f32(ld16(blk + 2));
-    } else if constexpr (T == kIQ2XXS) {
-        /* :758-822 */
-        const int sec = l >> 1, half = l & 1;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint8_t *codes = blk + 2 + 8 * g;
-            const uint32_t meta = ld32u(codes + 4);
-            const uint32_t grid = g_iq2xxs[2 * codes[sec] + half];
-            const uint32_t signs = sign_byte(meta >> (7 * sec)) >> (4 * half);
-            b.q[g] = negate_bytes(grid, byte_mask4(signs));
-            b.s[g] = 1 + 2 * (int)(meta >> 28);
-        }
-        b.d = 0.125f * f16_to_f32(ld16(blk));
-    } else if constexpr (T == kIQ2XS) {
-        /* :824-893 */
-        const int sec = l >> 1, half = l & 1;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t code = ld16(blk + 2 + 8 * g + 2 * sec);
-            const uint32_t grid = g_iq2xs[2 * (code & 511u) + half];
-            b.q[g] = negate_bytes(grid, byte_mask4(sign_byte(code >> 9) >> (4 * half)));
-            const uint32_t sc = blk[66 + g];
-            b.s[g] = 1 + 2 * (int)(hi ? sc >> 4 : sc & 15u);
-        }
-        b.d = 0.125f * f16_to_f32(ld16(blk));
-    } else if constexpr (T == kIQ2S) {
-        /* :664-756 */
-        const int sec = l >> 1, half = l & 1;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t index = blk[2 + 4 * g + sec] | (((uint32_t)blk[66 + g] << (8 - 2 * sec)) & 0x300u);
-            const uint32_t grid = g_iq2s[2 * index + half];
-            b.q[g] = negate_bytes(grid, byte_mask4((uint32_t)blk[34 + 4 * g + sec] >> (4 * half)));
-            const uint32_t sc = blk[74 + g];
-            b.s[g] = 1 + 2 * (int)(hi ? sc >> 4 : sc & 15u);
-        }
-        b.d = 0.125f * f16_to_f32(ld16(blk));
-    } else if constexpr (T == kIQ3XXS) {
-        /* :895-976 */
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t packed = ld32u(blk + 66 + 4 * g);
-            const uint32_t grid = g_iq3xxs[blk[2 + 8 * g + l]];
-            const uint32_t signs = sign_byte(packed >> (7 * (l >> 1))) >> (4 * (l & 1));
-            b.q[g] = negate_bytes(grid, byte_mask4(signs));
-            b.s[g] = 1 + 2 * (int)(packed >> 28);
-        }
-        b.d = 0.25f * f16_to_f32(ld16(blk));
-    } else if constexpr (T == kIQ3S) {
-        /* :978-1061 */
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t index = blk[2 + 8 * g + l] | (((uint32_t)(blk[66 + g] >> l) & 1u) << 8);
-            const uint32_t signs = (uint32_t)blk[74 + 4 * g + (l >> 1)] >> (4 * (l & 1));
-            b.q[g] = negate_bytes(g_iq3s[index], byte_mask4(signs));
-            b.s[g] = 1 + 2 * (int)((blk[106 + g / 2] >> (4 * (g & 1))) & 15u);
-        }
-        b.d = f16_to_f32(ld16(blk));
-    } else if constexpr (T == kIQ4XS) {
-        /* :1063-1127 */
-        const uint32_t scale_high = ld16(blk + 2);
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t qs = ld32a(blk + 8 + 16 * g + 4 * (l & 3));
-            b.q[g] = iq4nl_bytes(hi ? qs >> 4 : qs);
-            const int scale = (int)((blk[4 + g / 2] >> (4 * (g & 1))) & 15u) | (int)(((scale_high >> (2 * g)) & 3u) << 4);
-            b.s[g] = scale - 32;
-        }
-        b.d = f16_to_f32(ld16(blk));
-    } else if constexpr (T == kIQ4NL) {
-        /* :1129-1175: eight 18-byte blocks */
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t qs = ld32u(blk + 18 * g + 2 + 4 * (l & 3));
-            b.q[g] = iq4nl_bytes(hi ? qs >> 4 : qs);
-            b.s[g] = 1;
-            b.gd[g] = f16_to_f32(ld16(blk + 18 * g));
-        }
-    } else {
-        /* IQ1_S, :1177-1253 */
-        const int sec = l >> 1, half = l & 1;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t high = ld16(blk + 34 + 2 * g);
-            const uint32_t index = blk[2 + 4 * g + sec] | (((high >> (3 * sec)) & 7u) << 8);
-            b.q[g] = iq1s_grid[2 * index + half];
-            b.s[g] = 1 + 2 * (int)((high >> 12) & 7u);
-        }
-        b.d = f16_to_f32(ld16(blk));
-    }
-}
-
-/* the block's integer min (Q2_K, Q5_K) or correction (IQ1_S) term for one
- * token's Q8_K block */
-template <int T>
-__device__ __forceinline__ int block_extra(const uint8_t *blk, const uint8_t *xb)
-{
-    const int16_t *sums = reinterpret_cast<const int16_t *>(xb + 260);
-    int extra = 0;
-    if constexpr (T == kQ2K) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) extra += (blk[i] >> 4) * sums[i];
-    } else if constexpr (T == kQ5K) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            int sc0, m0, sc1, m1;
-            k4_scale_min(2 * c, blk + 4, sc0, m0);
-            k4_scale_min(2 * c + 1, blk + 4, sc1, m1);
-            extra += m0 * (sums[4 * c] + sums[4 * c + 1]) + m1 * (sums[4 * c + 2] + sums[4 * c + 3]);
-        }
-    } else if constexpr (T == kIQ1S) {
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t high = ld16(blk + 34 + 2 * g);
-            const int scale = 1 + 2 * (int)((high >> 12) & 7u);
-            extra += (high & 0x8000u ? -scale : scale) * (sums[2 * g] + sums[2 * g + 1]);
-        }
-    }
-    return extra;
-}
-
-template <int T>
-constexpr bool has_extra()
-{
-    return T == kQ2K || T == kQ5K || T == kIQ1S;
-}
 
 /* y[t * ldy + row] for t < MT: eight rows per wavefront, eight lanes per row */
 template <int T, int MT>

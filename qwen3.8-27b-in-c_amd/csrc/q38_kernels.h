@@ -78,6 +78,11 @@ bool format_takes_q8k(int type);
 bool format_row_decodable(int type);
 bool launch_gemm_format(int type, int m, const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy, uint32_t rows,
                         uint32_t nb, const void *grid, hipStream_t stream);
+/* q38_prompt.hip: the same products for a prompt batch of any length (from
+ * kWideMinTokens tokens on), and for row-major Q4_K and Q6_K; false for other
+ * types and for sizes past its 32-bit offsets */
+bool launch_gemm_prompt(int type, uint32_t tokens, const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy,
+                        uint32_t rows, uint32_t nb, const void *grid, hipStream_t stream);
 bool launch_gemm_float(int type, int m, const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows,
                        uint32_t width, hipStream_t stream);
 bool launch_row_decode(int type, const uint8_t *w, const uint32_t *ids, uint32_t first, uint32_t count,

@@ -1,0 +1,61 @@
+"""Prompt batches (9 tokens and more) of the row-major Q8_K formats on the
+matrix cores (q38hip_gemm_q8_k) against the oracle's one-token GEMV.  Bar:
+bit-identical fp32 outputs, since every integer sum is exact and the fp32
+chains keep their order.  Shapes sit at the edges of the 64-row x 64-token
+workgroup; the second input is Q8_K blocks with the extremes of the int8 and
+int16 fields and of the weights' packed fields, where the sums are largest."""
+import numpy as np
+import pytest
+
+import format_cases as fc
+from oracle import FORMAT_NAMES, IQ1_M, Q8K_DTYPE, Q8K_FORMATS
+
+pytestmark = [pytest.mark.gpu, pytest.mark.timeout(600)]
+
+TYPES = [t for t in Q8K_FORMATS if t != IQ1_M]
+
+
+def check(device, oracle, qtype, rows, width, data, q8, tokens):
+    import torch
+    import q38hip
+    nb = width // 256
+    want = np.stack([oracle.gemv(qtype, data, rows, q8[t * nb:(t + 1) * nb]) for t in range(tokens)])
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    got = q38hip.gemm_q8_k(dev(data), qtype, width, rows, dev(q8.view(np.uint8)), tokens).cpu().numpy()
+    wrong = int((got.view(np.uint32) != want.astype(np.float32).view(np.uint32)).sum())
+    assert wrong == 0, "%d of %d differ" % (wrong, got.size)
+
+
+@pytest.mark.parametrize("qtype", TYPES, ids=lambda t: FORMAT_NAMES[t])
+def test_prompt_batches_match_oracle(device, oracle, qtype):
+    rng = np.random.default_rng(700 + qtype)
+    # the last shape fills the chip with 128-token workgroups
+    for rows, width, tokens in ((1, 256, 24), (63, 512, 64), (65, 1280, 65), (130, 5120, 33), (64, 768, 131),
+                                (4100, 256, 9), (8200, 256, 130)):
+        print("%s rows=%d width=%d tokens=%d" % (FORMAT_NAMES[qtype], rows, width, tokens), flush=True)
+        data = fc.random_matrix(qtype, rows, width, rng)
+        q8 = oracle.quantize(rng.standard_normal(tokens * width).astype(np.float32))
+        check(device, oracle, qtype, rows, width, data, q8, tokens)
+
+
+@pytest.mark.parametrize("qtype", TYPES, ids=lambda t: FORMAT_NAMES[t])
+def test_prompt_extreme_fields_match_oracle(device, oracle, qtype):
+    rng = np.random.default_rng(800 + qtype)
+    rows, width, tokens = 40, 512, 26
+    data = fc.random_matrix(qtype, rows, width, rng).reshape(rows, -1)
+    scales = fc.random_matrix(qtype, rows, width, rng).reshape(rows, -1)
+    data[:20][data[:20] < 128] = 0      # rows of 0x00 and 0xff bytes
+    data[:20][data[:20] >= 128] = 255
+    fields = np.zeros(data.shape[1], bool)
+    block = fc.FORMATS[qtype][1]
+    for at in fc.SCALE_FIELDS[qtype]:   # finite super-scales in every row
+        for start in range(0, data.shape[1], block):
+            fields[start + at:start + at + 2] = True
+    data[:, fields] = scales[:, fields]
+    q8 = np.zeros(tokens * width // 256, dtype=Q8K_DTYPE)
+    q8["scale"] = rng.uniform(-0.1, 0.1, q8.size)
+    q8["quants"] = rng.choice([-128, -127, 127], q8["quants"].shape)
+    q8["quants"][:8] = 127              # whole blocks of one sign: the largest sums
+    q8["quants"][8:16] = -128
+    q8["sums"] = rng.choice([-32768, -2048, -1, 63, 2047, 32767], q8["sums"].shape)
+    check(device, oracle, qtype, rows, width, data.reshape(-1), q8, tokens)
