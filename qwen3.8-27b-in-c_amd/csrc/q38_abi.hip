@@ -260,13 +260,9 @@ int q38hip_gemm_f32(float *output, const float *input, uint32_t batch_size, uint
         q38::launch_fill_f32(output, (uint64_t)batch_size * rows, __builtin_nanf(""), s);
         return 1;
     }
-    for (uint32_t t0 = 0; t0 < batch_size;) {
-        const uint32_t n = std::min<uint32_t>(4, batch_size - t0);
-        if (!q38::launch_gemm_float((int)tensor->type, (int)n, tensor->data, input + (size_t)t0 * input_length,
-                                    output + (size_t)t0 * rows, rows, rows, (uint32_t)input_length, s))
-            return fail("unsupported float GEMM configuration");
-        t0 += n;
-    }
+    if (!q38::launch_gemm_float((int)tensor->type, batch_size, tensor->data, input, output, rows, rows,
+                                (uint32_t)input_length, s))
+        return fail("unsupported float GEMM configuration");
     return 1;
 }
 

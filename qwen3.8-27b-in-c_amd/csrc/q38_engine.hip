@@ -858,12 +858,8 @@ bool gemm_float(Q38Model *m, const DevTensor &w, uint32_t count, const float *xf
                 uint32_t rows, const uint8_t *wdata)
 {
     if (!xf) return report("float-input projection without its fp32 input");
-    for (uint32_t t0 = 0; t0 < count; t0 += 4) {
-        const uint32_t n = std::min<uint32_t>(4, count - t0);
-        if (!q38::launch_gemm_float((int)w.type, (int)n, wdata, xf + (size_t)t0 * w.width, out + (size_t)t0 * ldy, ldy,
-                                    rows, (uint32_t)w.width, m->stream))
-            return report("unsupported float GEMM configuration");
-    }
+    if (!q38::launch_gemm_float((int)w.type, count, wdata, xf, out, ldy, rows, (uint32_t)w.width, m->stream))
+        return report("unsupported float GEMM configuration");
     return true;
 }
 

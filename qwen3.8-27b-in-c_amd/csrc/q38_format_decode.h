@@ -334,6 +334,52 @@ __device__ __forceinline__ int block_extra(const uint8_t *blk, const uint8_t *xb
     return extra;
 }
 
+__device__ __forceinline__ float bf16_to_f32(uint32_t bits) { return __uint_as_float(bits << 16); }
+
+/* The weight expression of element i of a block (the first operand of its
+ * fmaf in the float dot), i < elements per block. */
+template <int T>
+__device__ __forceinline__ float element_weight(const uint8_t *blk, int i)
+{
+    if constexpr (T == kQ8_0) {
+        return __fmul_rn(f16_to_f32(ld16(blk)), (float)(int8_t)blk[2 + i]);
+    } else if constexpr (T == kIQ4NL) {
+        const uint32_t byte = blk[2 + (i & 15)];
+        return __fmul_rn(f16_to_f32(ld16(blk)), (float)kIq4nl[i < 16 ? byte & 15 : byte >> 4]);
+    } else if constexpr (T == kQ2K) {
+        const int s = i / 16, j = i % 16, half = s / 8, field = (s % 8) / 2, part = s % 2;
+        const float scale = __fmul_rn(f16_to_f32(ld16(blk + 80)), (float)(blk[s] & 15));
+        const float minimum = __fmul_rn(f16_to_f32(ld16(blk + 82)), (float)(blk[s] >> 4));
+        const int q = (blk[16 + 32 * half + 16 * part + j] >> (2 * field)) & 3;
+        return __fsub_rn(__fmul_rn(scale, (float)q), minimum);
+    } else if constexpr (T == kQ3K) {
+        const int g = i / 32, j = i % 32, half = g / 4, field = g % 4, si = 2 * g + j / 16;
+        const uint8_t *sc = blk + 96;
+        const int s = ((si < 8 ? sc[si] & 15 : sc[si - 8] >> 4) | (((sc[8 + si % 4] >> (2 * (si / 4))) & 3) << 4)) - 32;
+        const int q = ((blk[32 + 32 * half + j] >> (2 * field)) & 3) - ((blk[j] >> g) & 1 ? 0 : 4);
+        return __fmul_rn(__fmul_rn(f16_to_f32(ld16(blk + 108)), (float)s), (float)q);
+    } else if constexpr (T == kQ4K || T == kQ5K) {
+        constexpr bool five = T == kQ5K;
+        const int c = i / 64, upper = (i % 64) / 32, j = i % 32;
+        int sc, m;
+        k4_scale_min(2 * c + upper, blk + 4, sc, m);
+        const uint8_t byte = blk[(five ? 48 : 16) + 32 * c + j];
+        int q = upper ? byte >> 4 : byte & 15;
+        if (five && ((blk[16 + j] >> (2 * c + upper)) & 1)) q += 16;
+        const float dd = __fmul_rn(f16_to_f32(ld16(blk)), (float)sc);
+        const float mm = __fmul_rn(f16_to_f32(ld16(blk + 2)), (float)m);
+        return __fsub_rn(__fmul_rn(dd, (float)q), mm);
+    } else {
+        /* Q6_K: element 128 half + 32 k + i0 */
+        const int half = i / 128, k = (i % 128) / 32, i0 = i % 32;
+        const uint8_t *ql = blk + 64 * half, *qh = blk + 128 + 32 * half;
+        const uint8_t lowb = ql[i0 + (k & 1) * 32];
+        const int q = ((k < 2 ? lowb & 15 : lowb >> 4) | (((qh[i0] >> (2 * k)) & 3) << 4)) - 32;
+        const float ds = __fmul_rn(f16_to_f32(ld16(blk + 208)), (float)reinterpret_cast<const int8_t *>(blk + 192)[8 * half + i0 / 16 + 2 * k]);
+        return __fmul_rn(ds, (float)q);
+    }
+}
+
 template <int T>
 constexpr bool has_extra()
 {

@@ -1,8 +1,7 @@
-/* GEMV / small-M GEMM, float-input GEMV and row decode for the remaining
+/* GEMV / small-M GEMM and row decode for the remaining
  * GGUF matrix formats of the reference model (src/qwen38/qwen38_model.c:
  * 172-189): Q2_K, Q3_K, Q5_K, IQ2_XXS, IQ2_XS, IQ2_S, IQ3_XXS, IQ3_S,
- * IQ4_XS, IQ4_NL, IQ1_S against Q8_K activations, and F32, F16, BF16, Q8_0
- * (plus the K-quants and IQ4_NL) against fp32 activations.
+ * IQ4_XS, IQ4_NL, IQ1_S against Q8_K activations.
  *
  * Q8_K path.  Each of the reference's AVX2 kernels (qwen38_quant.c:510-1253,
  * 1636-1725) keeps eight fp32 lanes per row; for every super-block, lane l
@@ -16,10 +15,6 @@
  * ((a0 + a4) + (a2 + a6)) + ((a1 + a5) + (a3 + a7)); Q2_K and Q5_K add their
  * scalar min chain, IQ1_S 0.125 times its scalar correction sum, and IQ4_NL
  * applies one fp32 scale per 32-element group (eight FMAs per block).
- *
- * Float path (q38_dot_row, :2768-2810): one thread per row runs the row's
- * single fmaf chain in the reference's element order; the weight
- * expression of every element is rounded as the reference rounds it.
  *
  * Row decode (q38_tensor_row_f32, :3185-3223): F32 copied, F16 / BF16
  * converted; otherwise each element is the float dot of its block with a
@@ -117,186 +112,7 @@ void launch_format_m(int m, const uint8_t *w, const uint8_t *x, float *y, uint32
     }
 }
 
-/* ---- float path ------------------------------------------------------------ */
-
-__device__ __forceinline__ float bf16_to_f32(uint32_t bits) { return __uint_as_float(bits << 16); }
-
-/* The chain over one row for MT tokens: total_t = fmaf(w_e, x_t[e], total_t)
- * for every element e in the reference's order. */
-template <int T, int MT>
-__device__ __forceinline__ void float_chain(const uint8_t *row, const float *x, uint32_t width, float *total)
-{
-    auto step = [&](float wv, uint32_t e) {
-#pragma unroll
-        for (int t = 0; t < MT; ++t) total[t] = __builtin_fmaf(wv, x[(size_t)t * width + e], total[t]);
-    };
-    if constexpr (T == kF32) {
-        for (uint32_t e = 0; e < width; ++e) step(*reinterpret_cast<const float *>(row + 4 * (size_t)e), e);
-    } else if constexpr (T == kF16) {
-        for (uint32_t e = 0; e < width; ++e) step(f16_to_f32(ld16(row + 2 * (size_t)e)), e);
-    } else if constexpr (T == kBF16) {
-        for (uint32_t e = 0; e < width; ++e) step(bf16_to_f32(ld16(row + 2 * (size_t)e)), e);
-    } else if constexpr (T == kQ8_0) {
-        /* :496-507 */
-        for (uint32_t base = 0; base < width; base += 32, row += 34) {
-            const float d = f16_to_f32(ld16(row));
-            for (int i = 0; i < 32; ++i) step(__fmul_rn(d, (float)(int8_t)row[2 + i]), base + i);
-        }
-    } else if constexpr (T == kIQ4NL) {
-        /* :2796-2807 */
-        for (uint32_t base = 0; base < width; base += 32, row += 18) {
-            const float d = f16_to_f32(ld16(row));
-            for (int j = 0; j < 16; ++j) {
-                step(__fmul_rn(d, (float)kIq4nl[row[2 + j] & 15]), base + j);
-                step(__fmul_rn(d, (float)kIq4nl[row[2 + j] >> 4]), base + 16 + j);
-            }
-        }
-    } else if constexpr (T == kQ2K) {
-        /* :331-362 */
-        for (uint32_t base = 0; base < width; base += 256, row += 84) {
-            const float d = f16_to_f32(ld16(row + 80)), dmin = f16_to_f32(ld16(row + 82));
-            for (int i = 0; i < 16; ++i) {
-                const float scale = __fmul_rn(d, (float)(row[i] & 15)), minimum = __fmul_rn(dmin, (float)(row[i] >> 4));
-                const int half = i / 8, field = (i % 8) / 2, part = i % 2;
-                for (int j = 0; j < 16; ++j) {
-                    const int q = (row[16 + 32 * half + 16 * part + j] >> (2 * field)) & 3;
-                    step(__fsub_rn(__fmul_rn(scale, (float)q), minimum), base + 16 * i + j);
-                }
-            }
-        }
-    } else if constexpr (T == kQ3K) {
-        /* :364-394 */
-        for (uint32_t base = 0; base < width; base += 256, row += 110) {
-            const float d = f16_to_f32(ld16(row + 108));
-            const uint8_t *sc = row + 96;
-            for (int g = 0; g < 8; ++g) {
-                const int half = g / 4, field = g % 4;
-                for (int j = 0; j < 32; ++j) {
-                    const int i = 2 * g + j / 16;
-                    const int s = ((i < 8 ? sc[i] & 15 : sc[i - 8] >> 4) | (((sc[8 + i % 4] >> (2 * (i / 4))) & 3) << 4)) - 32;
-                    const int q = ((row[32 + 32 * half + j] >> (2 * field)) & 3) - ((row[j] >> g) & 1 ? 0 : 4);
-                    step(__fmul_rn(__fmul_rn(d, (float)s), (float)q), base + 32 * g + j);
-                }
-            }
-        }
-    } else if constexpr (T == kQ4K || T == kQ5K) {
-        /* :396-464 */
-        constexpr bool five = T == kQ5K;
-        for (uint32_t base = 0; base < width; base += 256, row += five ? 176 : 144) {
-            const float d = f16_to_f32(ld16(row)), dmin = f16_to_f32(ld16(row + 2));
-            const uint8_t *qh = row + 16, *qs = row + (five ? 48 : 16);
-            for (int c = 0; c < 4; ++c) {
-                int sc0, m0, sc1, m1;
-                k4_scale_min(2 * c, row + 4, sc0, m0);
-                k4_scale_min(2 * c + 1, row + 4, sc1, m1);
-                const float d0 = __fmul_rn(d, (float)sc0), mm0 = __fmul_rn(dmin, (float)m0);
-                const float d1 = __fmul_rn(d, (float)sc1), mm1 = __fmul_rn(dmin, (float)m1);
-                for (int i = 0; i < 32; ++i) {
-                    const int q = (qs[32 * c + i] & 15) + (five && ((qh[i] >> (2 * c)) & 1) ? 16 : 0);
-                    step(__fsub_rn(__fmul_rn(d0, (float)q), mm0), base + 64 * c + i);
-                }
-                for (int i = 0; i < 32; ++i) {
-                    const int q = (qs[32 * c + i] >> 4) + (five && ((qh[i] >> (2 * c + 1)) & 1) ? 16 : 0);
-                    step(__fsub_rn(__fmul_rn(d1, (float)q), mm1), base + 64 * c + 32 + i);
-                }
-            }
-        }
-    } else {
-        /* Q6_K, :466-494 */
-        for (uint32_t base = 0; base < width; base += 256, row += 210) {
-            const float d = f16_to_f32(ld16(row + 208));
-            const int8_t *scales = reinterpret_cast<const int8_t *>(row + 192);
-            for (int half = 0; half < 2; ++half) {
-                const uint8_t *ql = row + 64 * half, *qh = row + 128 + 32 * half;
-                const int8_t *sc = scales + 8 * half;
-                for (int i = 0; i < 32; ++i) {
-                    const int q[4] = {((ql[i] & 15) | ((qh[i] & 3) << 4)) - 32,
-                                      ((ql[i + 32] & 15) | (((qh[i] >> 2) & 3) << 4)) - 32,
-                                      ((ql[i] >> 4) | (((qh[i] >> 4) & 3) << 4)) - 32,
-                                      ((ql[i + 32] >> 4) | (((qh[i] >> 6) & 3) << 4)) - 32};
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        step(__fmul_rn(__fmul_rn(d, (float)sc[i / 16 + 2 * k]), (float)q[k]),
-                             base + 128 * half + 32 * k + i);
-                }
-            }
-        }
-    }
-}
-
-template <int T, int MT>
-__global__ __launch_bounds__(256) void gemv_float_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x,
-                                                         float *__restrict__ y, uint32_t ldy, uint32_t rows,
-                                                         uint32_t width, uint64_t row_bytes)
-{
-    const uint32_t row = blockIdx.x * 256u + threadIdx.x;
-    if (row >= rows) return;
-    float total[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) total[t] = 0.0f;
-    float_chain<T, MT>(w + row * row_bytes, x, width, total);
-#pragma unroll
-    for (int t = 0; t < MT; ++t) y[(size_t)t * ldy + row] = total[t];
-}
-
-template <int T>
-void launch_float_m(int m, const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows, uint32_t width,
-                    uint64_t row_bytes, hipStream_t stream)
-{
-    const dim3 grid((rows + 255) / 256), block(256);
-    switch (m) {
-    case 1: hipLaunchKernelGGL((gemv_float_kernel<T, 1>), grid, block, 0, stream, w, x, y, ldy, rows, width, row_bytes); break;
-    case 2: hipLaunchKernelGGL((gemv_float_kernel<T, 2>), grid, block, 0, stream, w, x, y, ldy, rows, width, row_bytes); break;
-    case 3: hipLaunchKernelGGL((gemv_float_kernel<T, 3>), grid, block, 0, stream, w, x, y, ldy, rows, width, row_bytes); break;
-    default: hipLaunchKernelGGL((gemv_float_kernel<T, 4>), grid, block, 0, stream, w, x, y, ldy, rows, width, row_bytes); break;
-    }
-}
-
 /* ---- row decode ------------------------------------------------------------ */
-
-/* The weight expression of element i of a block (the first operand of its
- * fmaf in the float dot), i < elements per block. */
-template <int T>
-__device__ __forceinline__ float element_weight(const uint8_t *blk, int i)
-{
-    if constexpr (T == kQ8_0) {
-        return __fmul_rn(f16_to_f32(ld16(blk)), (float)(int8_t)blk[2 + i]);
-    } else if constexpr (T == kIQ4NL) {
-        const uint32_t byte = blk[2 + (i & 15)];
-        return __fmul_rn(f16_to_f32(ld16(blk)), (float)kIq4nl[i < 16 ? byte & 15 : byte >> 4]);
-    } else if constexpr (T == kQ2K) {
-        const int s = i / 16, j = i % 16, half = s / 8, field = (s % 8) / 2, part = s % 2;
-        const float scale = __fmul_rn(f16_to_f32(ld16(blk + 80)), (float)(blk[s] & 15));
-        const float minimum = __fmul_rn(f16_to_f32(ld16(blk + 82)), (float)(blk[s] >> 4));
-        const int q = (blk[16 + 32 * half + 16 * part + j] >> (2 * field)) & 3;
-        return __fsub_rn(__fmul_rn(scale, (float)q), minimum);
-    } else if constexpr (T == kQ3K) {
-        const int g = i / 32, j = i % 32, half = g / 4, field = g % 4, si = 2 * g + j / 16;
-        const uint8_t *sc = blk + 96;
-        const int s = ((si < 8 ? sc[si] & 15 : sc[si - 8] >> 4) | (((sc[8 + si % 4] >> (2 * (si / 4))) & 3) << 4)) - 32;
-        const int q = ((blk[32 + 32 * half + j] >> (2 * field)) & 3) - ((blk[j] >> g) & 1 ? 0 : 4);
-        return __fmul_rn(__fmul_rn(f16_to_f32(ld16(blk + 108)), (float)s), (float)q);
-    } else if constexpr (T == kQ4K || T == kQ5K) {
-        constexpr bool five = T == kQ5K;
-        const int c = i / 64, upper = (i % 64) / 32, j = i % 32;
-        int sc, m;
-        k4_scale_min(2 * c + upper, blk + 4, sc, m);
-        const uint8_t byte = blk[(five ? 48 : 16) + 32 * c + j];
-        int q = upper ? byte >> 4 : byte & 15;
-        if (five && ((blk[16 + j] >> (2 * c + upper)) & 1)) q += 16;
-        const float dd = __fmul_rn(f16_to_f32(ld16(blk)), (float)sc);
-        const float mm = __fmul_rn(f16_to_f32(ld16(blk + 2)), (float)m);
-        return __fsub_rn(__fmul_rn(dd, (float)q), mm);
-    } else {
-        /* Q6_K: element 128 half + 32 k + i0 */
-        const int half = i / 128, k = (i % 128) / 32, i0 = i % 32;
-        const uint8_t *ql = blk + 64 * half, *qh = blk + 128 + 32 * half;
-        const uint8_t lowb = ql[i0 + (k & 1) * 32];
-        const int q = ((k < 2 ? lowb & 15 : lowb >> 4) | (((qh[i0] >> (2 * k)) & 3) << 4)) - 32;
-        const float ds = __fmul_rn(f16_to_f32(ld16(blk + 208)), (float)reinterpret_cast<const int8_t *>(blk + 192)[8 * half + i0 / 16 + 2 * k]);
-        return __fmul_rn(ds, (float)q);
-    }
-}
 
 /* rows[r] of the matrix into out[r * width ..]; the row index of output row
  * r is ids[r] (a token id) when ids is set, else first + r.  One workgroup
@@ -426,27 +242,6 @@ bool launch_gemm_format(int type, int m, const uint8_t *w, const uint8_t *x, flo
         if (!grid) return false;
         launch_format_m<kIQ1S>(m, w, x, y, ldy, rows, nb, grid, stream);
         return true;
-    default: return false;
-    }
-}
-
-bool launch_gemm_float(int type, int m, const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows,
-                       uint32_t width, hipStream_t stream)
-{
-    uint32_t e = 0, b = 0;
-    if (m < 1 || m > 4 || ldy < rows || !rows || !format_block_shape(type, &e, &b) || width % e) return false;
-    const uint64_t row_bytes = (uint64_t)width / e * b;
-    switch (type) {
-    case kF32: launch_float_m<kF32>(m, w, x, y, ldy, rows, width, row_bytes, stream); return true;
-    case kF16: launch_float_m<kF16>(m, w, x, y, ldy, rows, width, row_bytes, stream); return true;
-    case kBF16: launch_float_m<kBF16>(m, w, x, y, ldy, rows, width, row_bytes, stream); return true;
-    case kQ8_0: launch_float_m<kQ8_0>(m, w, x, y, ldy, rows, width, row_bytes, stream); return true;
-    case kIQ4NL: launch_float_m<kIQ4NL>(m, w, x, y, ldy, rows, width, row_bytes, stream); return true;
-    case kQ2K: launch_float_m<kQ2K>(m, w, x, y, ldy, rows, width, row_bytes, stream); return true;
-    case kQ3K: launch_float_m<kQ3K>(m, w, x, y, ldy, rows, width, row_bytes, stream); return true;
-    case kQ4K: launch_float_m<kQ4K>(m, w, x, y, ldy, rows, width, row_bytes, stream); return true;
-    case kQ5K: launch_float_m<kQ5K>(m, w, x, y, ldy, rows, width, row_bytes, stream); return true;
-    case kQ6K: launch_float_m<kQ6K>(m, w, x, y, ldy, rows, width, row_bytes, stream); return true;
     default: return false;
     }
 }

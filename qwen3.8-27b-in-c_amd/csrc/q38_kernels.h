@@ -68,9 +68,9 @@ bool launch_gemm_ld(int type, int m, const uint8_t *w, const uint8_t *x, float *
  * activations (else fp32).  launch_gemm_format: y[t * ldy + row] for t < m
  * (1..8) against Q8_K activations, for Q2_K, Q3_K, Q5_K, IQ2_XXS, IQ2_XS,
  * IQ2_S, IQ3_XXS, IQ3_S, IQ4_XS, IQ4_NL and IQ1_S (`grid`: the IQ1_M/IQ1_S
- * codebook as 2048 x 8 int8); false for other types.  launch_gemm_float:
- * the same against fp32 activations x[t * width + e] (m 1..4) for F32, F16,
- * BF16, Q8_0, IQ4_NL and Q2_K..Q6_K.  launch_row_decode: rows of such a
+ * codebook as 2048 x 8 int8); false for other types.  launch_gemm_float
+ * (q38_float.hip): the same against fp32 activations x[t * width + e] (any m)
+ * for F32, F16, BF16, Q8_0, IQ4_NL and Q2_K..Q6_K.  launch_row_decode: rows of such a
  * matrix as fp32 (q38_tensor_row_f32), output row r from matrix row ids[r]
  * (clamped below `limit`) or first + r. */
 bool format_block_shape(int type, uint32_t *elements, uint32_t *bytes);
@@ -83,7 +83,7 @@ bool launch_gemm_format(int type, int m, const uint8_t *w, const uint8_t *x, flo
  * types and for sizes past its 32-bit offsets */
 bool launch_gemm_prompt(int type, uint32_t tokens, const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy,
                         uint32_t rows, uint32_t nb, const void *grid, hipStream_t stream);
-bool launch_gemm_float(int type, int m, const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows,
+bool launch_gemm_float(int type, uint32_t m, const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows,
                        uint32_t width, hipStream_t stream);
 bool launch_row_decode(int type, const uint8_t *w, const uint32_t *ids, uint32_t first, uint32_t count,
                        uint32_t limit, float *out, uint32_t width, hipStream_t stream);

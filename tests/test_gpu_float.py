@@ -1,0 +1,52 @@
+"""Matrices against fp32 activations (q38hip_gemm_f32) at the edges of the
+kernel's 64-row workgroups, 64-column stages and token tiles, against the
+oracle's one-token chain (orc_format_gemv_f32).  Bar: bit-identical outputs,
+the chain having one order.  F32, F16 and BF16 take any width; an infinite
+weight or activation must reach exactly its own outputs."""
+import numpy as np
+import pytest
+
+import format_cases as fc
+from oracle import BF16, F16, F32, FORMAT_NAMES, IQ4_NL, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0
+
+pytestmark = [pytest.mark.gpu, pytest.mark.timeout(600)]
+
+# (rows, width, tokens); widths are rounded up to the format's block
+SHAPES = ((1, 1, 1), (63, 67, 2), (65, 130, 3), (64, 64, 4), (5, 255, 5), (70, 320, 9), (66, 1000, 33), (64, 192, 66),
+          (96, 5120, 1), (130, 769, 1))
+
+
+def run(device, oracle, qtype, rows, width, tokens, data, x):
+    import torch
+    import q38hip
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    got = q38hip.gemm_f32(dev(data), qtype, width, rows, dev(x)).cpu().numpy()
+    want = np.stack([oracle.gemv_f32(qtype, data, rows, x[t]) for t in range(tokens)])
+    finite = np.isfinite(want)
+    assert np.array_equal(finite, np.isfinite(got)) and np.array_equal(np.isnan(want), np.isnan(got))
+    assert int((got.view(np.uint32) != want.view(np.uint32))[~np.isnan(want)].sum()) == 0
+
+
+@pytest.mark.parametrize("qtype", (F32, F16, BF16, Q8_0, IQ4_NL, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K),
+                         ids=lambda t: FORMAT_NAMES[t])
+def test_float_gemm_edges(device, oracle, qtype):
+    rng = np.random.default_rng(900 + qtype)
+    elements = fc.FORMATS[qtype][0]
+    for rows, width, tokens in SHAPES:
+        width = -(-width // elements) * elements
+        print("%s rows=%d width=%d tokens=%d" % (FORMAT_NAMES[qtype], rows, width, tokens), flush=True)
+        data = fc.random_matrix(qtype, rows, width, rng)
+        run(device, oracle, qtype, rows, width, tokens, data, rng.standard_normal((tokens, width)).astype(np.float32))
+
+
+@pytest.mark.parametrize("qtype", (F32, F16, BF16), ids=lambda t: FORMAT_NAMES[t])
+def test_float_gemm_non_finite(device, oracle, qtype):
+    rng = np.random.default_rng(950 + qtype)
+    rows, width, tokens = 67, 131, 5
+    data = fc.random_matrix(qtype, rows, width, rng)
+    bits = {F32: (np.uint32, 0x7F800000), F16: (np.uint16, 0x7C00), BF16: (np.uint16, 0x7F80)}[qtype]
+    cells = data.view(bits[0]).reshape(rows, width)
+    cells[3, 130], cells[66, 0] = bits[1], bits[1]
+    x = rng.standard_normal((tokens, width)).astype(np.float32)
+    x[2, 64], x[4, 130] = -np.inf, np.nan
+    run(device, oracle, qtype, rows, width, tokens, data, x)
