@@ -57,11 +57,25 @@ __device__ __forceinline__ uint32_t ld16(const uint8_t *p)
 {
     return (uint32_t)p[0] | (uint32_t)p[1] << 8;
 }
-/* 4 bytes at a 2-byte aligned address */
-__device__ __forceinline__ uint32_t ld32u(const uint8_t *p)
+/* N dwords at a 2-byte aligned address (one load: the hardware takes
+ * unaligned dwords) */
+template <int N>
+struct Dwords {
+    uint32_t v[N];
+};
+template <int N>
+__device__ __forceinline__ Dwords<N> ldn(const uint8_t *p)
 {
-    const uint16_t *h = reinterpret_cast<const uint16_t *>(p);
-    return (uint32_t)h[0] | (uint32_t)h[1] << 16;
+    Dwords<N> r;
+    __builtin_memcpy(&r, p, 4 * N);
+    return r;
+}
+__device__ __forceinline__ uint32_t ld32u(const uint8_t *p) { return ldn<1>(p).v[0]; }
+/* byte k of an array of dwords */
+template <int N>
+__device__ __forceinline__ uint32_t byte_of(const Dwords<N> &a, int k)
+{
+    return (a.v[k >> 2] >> (8 * (k & 3))) & 255u;
 }
 __device__ __forceinline__ uint32_t ld32a(const uint8_t *p) { return *reinterpret_cast<const uint32_t *>(p); }
 
@@ -119,7 +133,7 @@ struct LaneBlock {
 };
 
 template <int T>
-__device__ __forceinline__ uint32_t block_bytes()
+constexpr uint32_t block_bytes()
 {
     switch (T) {
     case kQ2K: return 84;
@@ -138,68 +152,103 @@ __device__ __forceinline__ uint32_t block_bytes()
     }
 }
 
+/* the 6-bit scales of the eight sub-blocks of Q4_K / Q5_K from the 12 packed
+ * bytes, four per dword (sc) and the mins alike (m) (qwen38_quant.c:131-143) */
+struct K4Scales {
+    uint32_t sc[2], m[2];
+};
+__device__ __forceinline__ K4Scales k4_scales(const uint8_t *p)
+{
+    const Dwords<3> w = ldn<3>(p);
+    return {{w.v[0] & 0x3f3f3f3fu, (w.v[2] & 0x0f0f0f0fu) | ((w.v[0] >> 2) & 0x30303030u)},
+            {w.v[1] & 0x3f3f3f3fu, ((w.v[2] >> 4) & 0x0f0f0f0fu) | ((w.v[1] >> 2) & 0x30303030u)}};
+}
+
+/* the codebook of an IQ format as dwords: entries and their count (IQ1_S
+ * takes the caller's table of 2048 x 8 int8) */
 template <int T>
-__device__ __forceinline__ void decode_lane(const uint8_t *blk, int l, const uint32_t *iq1s_grid, LaneBlock &b)
+constexpr int table_dwords()
+{
+    switch (T) {
+    case kIQ2XXS: return 512;
+    case kIQ2XS: return 1024;
+    case kIQ2S: return 2048;
+    case kIQ3XXS: return 256;
+    case kIQ3S: return 512;
+    case kIQ1S: return 4096;
+    default: return 0;
+    }
+}
+template <int T>
+__device__ __forceinline__ const uint32_t *table_of(const uint32_t *iq1s)
+{
+    if constexpr (T == kIQ2XXS) return g_iq2xxs;
+    else if constexpr (T == kIQ2XS) return g_iq2xs;
+    else if constexpr (T == kIQ2S) return g_iq2s;
+    else if constexpr (T == kIQ3XXS) return g_iq3xxs;
+    else if constexpr (T == kIQ3S) return g_iq3s;
+    else return iq1s;
+}
+
+/* lane l's share of the block at blk; `table` is the format's codebook
+ * (table_of, or a copy of it).  Header fields are loaded as whole dwords. */
+template <int T>
+__device__ __forceinline__ void decode_lane(const uint8_t *blk, int l, const uint32_t *table, LaneBlock &b)
 {
     const int hi = l >= 4;
     if constexpr (T == kQ2K) {
         /* qwen38_quant.c:510-585 */
         const uint32_t d0 = ld32a(blk + 16 + 4 * l), d1 = ld32a(blk + 48 + 4 * l);
+        const Dwords<4> sc = ldn<4>(blk);
 #pragma unroll
         for (int g = 0; g < 8; ++g) {
             b.q[g] = ((g < 4 ? d0 : d1) >> (2 * (g & 3))) & 0x03030303u;
-            b.s[g] = blk[2 * g + hi] & 15;
+            b.s[g] = (sc.v[g >> 1] >> (16 * (g & 1) + 8 * hi)) & 15;
         }
-        b.d = f16_to_f32(ld16(blk + 80));
-        b.dmin = f16_to_f32(ld16(blk + 82));
+        const uint32_t dd = ld32a(blk + 80);
+        b.d = f16_to_f32(dd);
+        b.dmin = f16_to_f32(dd >> 16);
     } else if constexpr (T == kQ3K) {
-        /* :587-662; scales :319-329 */
+        /* :587-662; scales :319-329: low nibbles of bytes 0..7, their high
+         * nibbles, and two high bits each in bytes 8..11 */
         const uint32_t hm = ld32u(blk + 4 * l);
         const uint32_t d0 = ld32u(blk + 32 + 4 * l), d1 = ld32u(blk + 64 + 4 * l);
-        const uint8_t *sc = blk + 96;
+        const Dwords<3> sc = ldn<3>(blk + 96);
+        const uint32_t six[4] = {(sc.v[0] & 0x0f0f0f0fu) | (sc.v[2] << 4 & 0x30303030u),
+                                 (sc.v[1] & 0x0f0f0f0fu) | (sc.v[2] << 2 & 0x30303030u),
+                                 (sc.v[0] >> 4 & 0x0f0f0f0fu) | (sc.v[2] & 0x30303030u),
+                                 (sc.v[1] >> 4 & 0x0f0f0f0fu) | (sc.v[2] >> 2 & 0x30303030u)};
 #pragma unroll
         for (int g = 0; g < 8; ++g) {
             const uint32_t low = ((g < 4 ? d0 : d1) >> (2 * (g & 3))) & 0x03030303u;
             const uint32_t absent = ~(hm >> g) & 0x01010101u;
             b.q[g] = low + absent * 0xfcu;   /* minus 4 where the high bit is clear */
-            const int i = 2 * g + hi;
-            const int lo4 = i < 8 ? sc[i] & 15 : sc[i - 8] >> 4;
-            const int hi2 = (sc[8 + i % 4] >> (2 * (i / 4))) & 3;
-            b.s[g] = (lo4 | hi2 << 4) - 32;
+            b.s[g] = (int)((six[g >> 1] >> (16 * (g & 1) + 8 * hi)) & 63u) - 32;
         }
         b.d = f16_to_f32(ld16(blk + 108));
-    } else if constexpr (T == kQ5K) {
-        /* :1636-1725 */
-        const uint32_t qh = ld32a(blk + 16 + 4 * l);
+    } else if constexpr (T == kQ5K || T == kQ4K) {
+        /* :1636-1725, :1546-1634 */
+        const uint32_t qh = T == kQ5K ? ld32a(blk + 16 + 4 * l) : 0u;
+        const K4Scales k4 = k4_scales(blk + 4);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const uint32_t qs = ld32a(blk + 48 + 32 * c + 4 * l);
-            b.q[2 * c] = (qs & 0x0f0f0f0fu) + (((qh >> (2 * c)) & 0x01010101u) << 4);
-            b.q[2 * c + 1] = ((qs >> 4) & 0x0f0f0f0fu) + (((qh >> (2 * c + 1)) & 0x01010101u) << 4);
-            int sc0, m0, sc1, m1;
-            k4_scale_min(2 * c, blk + 4, sc0, m0);
-            k4_scale_min(2 * c + 1, blk + 4, sc1, m1);
-            b.s[2 * c] = sc0;
-            b.s[2 * c + 1] = sc1;
-        }
-        b.d = f16_to_f32(ld16(blk));
-        b.dmin = f16_to_f32(ld16(blk + 2));
-    } else if constexpr (T == kQ4K) {
-        /* :1546-1634 */
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const uint32_t qs = ld32a(blk + 16 + 32 * c + 4 * l);
+            const uint32_t qs = ld32a(blk + (T == kQ5K ? 48 : 16) + 32 * c + 4 * l);
             b.q[2 * c] = qs & 0x0f0f0f0fu;
             b.q[2 * c + 1] = (qs >> 4) & 0x0f0f0f0fu;
-            int m;
-            k4_scale_min(2 * c, blk + 4, b.s[2 * c], m);
-            k4_scale_min(2 * c + 1, blk + 4, b.s[2 * c + 1], m);
+            if constexpr (T == kQ5K) {
+                b.q[2 * c] |= ((qh >> (2 * c)) & 0x01010101u) << 4;
+                b.q[2 * c + 1] |= ((qh >> (2 * c + 1)) & 0x01010101u) << 4;
+            }
         }
-        b.d = f16_to_f32(ld16(blk));
-        b.dmin = f16_to_f32(ld16(blk + 2));
+#pragma unroll
+        for (int g = 0; g < 8; ++g) b.s[g] = (k4.sc[g >> 2] >> (8 * (g & 3))) & 255u;
+        const uint32_t dd = ld32a(blk);
+        b.d = f16_to_f32(dd);
+        b.dmin = f16_to_f32(dd >> 16);
     } else if constexpr (T == kQ6K) {
         /* :1727-1814, the quants minus 32 (the reference's unsigned form
          * subtracts the 32s through the activation sums) */
+        const Dwords<4> sc = ldn<4>(blk + 192);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const uint32_t low[2] = {ld32u(blk + 64 * h + 4 * l), ld32u(blk + 64 * h + 32 + 4 * l)};
@@ -209,7 +258,7 @@ __device__ __forceinline__ void decode_lane(const uint8_t *blk, int l, const uin
                 const uint32_t v = ((low[j & 1] >> (j < 2 ? 0 : 4)) & 0x0f0f0f0fu) | ((high >> (2 * j)) & 0x03030303u) << 4;
                 const uint32_t x = v ^ 0x20202020u;   /* 6-bit two's complement of v - 32 */
                 b.q[4 * h + j] = x | ((x >> 5) & 0x01010101u) * 0xc0u;
-                b.s[4 * h + j] = (int8_t)blk[192 + 8 * h + 2 * j + hi];
+                b.s[4 * h + j] = (int8_t)(sc.v[2 * h + (j >> 1)] >> (16 * (j & 1) + 8 * hi));
             }
         }
         b.d = f16_to_f32(ld16(blk + 208));
@@ -218,70 +267,84 @@ __device__ __forceinline__ void decode_lane(const uint8_t *blk, int l, const uin
         const int sec = l >> 1, half = l & 1;
 #pragma unroll
         for (int g = 0; g < 8; ++g) {
-            const uint8_t *codes = blk + 2 + 8 * g;
-            const uint32_t meta = ld32u(codes + 4);
-            const uint32_t grid = g_iq2xxs[2 * codes[sec] + half];
-            const uint32_t signs = sign_byte(meta >> (7 * sec)) >> (4 * half);
+            const Dwords<2> w = ldn<2>(blk + 2 + 8 * g);   /* four codes; sign indices and scale */
+            const uint32_t grid = table[2 * ((w.v[0] >> (8 * sec)) & 255u) + half];
+            const uint32_t signs = sign_byte(w.v[1] >> (7 * sec)) >> (4 * half);
             b.q[g] = negate_bytes(grid, byte_mask4(signs));
-            b.s[g] = 1 + 2 * (int)(meta >> 28);
+            b.s[g] = 1 + 2 * (int)(w.v[1] >> 28);
         }
         b.d = 0.125f * f16_to_f32(ld16(blk));
     } else if constexpr (T == kIQ2XS) {
         /* :824-893 */
         const int sec = l >> 1, half = l & 1;
+        const Dwords<2> sc = ldn<2>(blk + 66);
 #pragma unroll
         for (int g = 0; g < 8; ++g) {
             const uint32_t code = ld16(blk + 2 + 8 * g + 2 * sec);
-            const uint32_t grid = g_iq2xs[2 * (code & 511u) + half];
+            const uint32_t grid = table[2 * (code & 511u) + half];
             b.q[g] = negate_bytes(grid, byte_mask4(sign_byte(code >> 9) >> (4 * half)));
-            const uint32_t sc = blk[66 + g];
-            b.s[g] = 1 + 2 * (int)(hi ? sc >> 4 : sc & 15u);
+            b.s[g] = 1 + 2 * (int)((sc.v[g >> 2] >> (8 * (g & 3) + 4 * hi)) & 15u);
         }
         b.d = 0.125f * f16_to_f32(ld16(blk));
     } else if constexpr (T == kIQ2S) {
         /* :664-756 */
         const int sec = l >> 1, half = l & 1;
+        const Dwords<4> qh_sc = ldn<4>(blk + 66);
 #pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t index = blk[2 + 4 * g + sec] | (((uint32_t)blk[66 + g] << (8 - 2 * sec)) & 0x300u);
-            const uint32_t grid = g_iq2s[2 * index + half];
-            b.q[g] = negate_bytes(grid, byte_mask4((uint32_t)blk[34 + 4 * g + sec] >> (4 * half)));
-            const uint32_t sc = blk[74 + g];
-            b.s[g] = 1 + 2 * (int)(hi ? sc >> 4 : sc & 15u);
+        for (int p = 0; p < 2; ++p) {
+            const Dwords<4> codes = ldn<4>(blk + 2 + 16 * p), sg = ldn<4>(blk + 34 + 16 * p);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int g = 4 * p + i;
+                const uint32_t index = ((codes.v[i] >> (8 * sec)) & 255u) | ((byte_of(qh_sc, g) << (8 - 2 * sec)) & 0x300u);
+                const uint32_t grid = table[2 * index + half];
+                b.q[g] = negate_bytes(grid, byte_mask4(sg.v[i] >> (8 * sec + 4 * half)));
+                b.s[g] = 1 + 2 * (int)((byte_of(qh_sc, 8 + g) >> (4 * hi)) & 15u);
+            }
         }
         b.d = 0.125f * f16_to_f32(ld16(blk));
     } else if constexpr (T == kIQ3XXS) {
         /* :895-976 */
 #pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t packed = ld32u(blk + 66 + 4 * g);
-            const uint32_t grid = g_iq3xxs[blk[2 + 8 * g + l]];
-            const uint32_t signs = sign_byte(packed >> (7 * (l >> 1))) >> (4 * (l & 1));
-            b.q[g] = negate_bytes(grid, byte_mask4(signs));
-            b.s[g] = 1 + 2 * (int)(packed >> 28);
+        for (int p = 0; p < 2; ++p) {
+            const Dwords<4> meta = ldn<4>(blk + 66 + 16 * p);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int g = 4 * p + i;
+                const uint32_t grid = table[blk[2 + 8 * g + l]];
+                const uint32_t signs = sign_byte(meta.v[i] >> (7 * (l >> 1))) >> (4 * (l & 1));
+                b.q[g] = negate_bytes(grid, byte_mask4(signs));
+                b.s[g] = 1 + 2 * (int)(meta.v[i] >> 28);
+            }
         }
         b.d = 0.25f * f16_to_f32(ld16(blk));
     } else if constexpr (T == kIQ3S) {
         /* :978-1061 */
+        const Dwords<2> qh = ldn<2>(blk + 66);
+        const uint32_t sc = ld32u(blk + 106);
 #pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t index = blk[2 + 8 * g + l] | (((uint32_t)(blk[66 + g] >> l) & 1u) << 8);
-            const uint32_t signs = (uint32_t)blk[74 + 4 * g + (l >> 1)] >> (4 * (l & 1));
-            b.q[g] = negate_bytes(g_iq3s[index], byte_mask4(signs));
-            b.s[g] = 1 + 2 * (int)((blk[106 + g / 2] >> (4 * (g & 1))) & 15u);
+        for (int p = 0; p < 2; ++p) {
+            const Dwords<4> sg = ldn<4>(blk + 74 + 16 * p);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int g = 4 * p + i;
+                const uint32_t index = blk[2 + 8 * g + l] | (((byte_of(qh, g) >> l) & 1u) << 8);
+                const uint32_t signs = sg.v[i] >> (8 * (l >> 1) + 4 * (l & 1));
+                b.q[g] = negate_bytes(table[index], byte_mask4(signs));
+                b.s[g] = 1 + 2 * (int)((sc >> (4 * g)) & 15u);
+            }
         }
         b.d = f16_to_f32(ld16(blk));
     } else if constexpr (T == kIQ4XS) {
         /* :1063-1127 */
-        const uint32_t scale_high = ld16(blk + 2);
+        const Dwords<2> head = ldn<2>(blk);   /* d, scale high bits; scale low nibbles */
 #pragma unroll
         for (int g = 0; g < 8; ++g) {
             const uint32_t qs = ld32a(blk + 8 + 16 * g + 4 * (l & 3));
             b.q[g] = iq4nl_bytes(hi ? qs >> 4 : qs);
-            const int scale = (int)((blk[4 + g / 2] >> (4 * (g & 1))) & 15u) | (int)(((scale_high >> (2 * g)) & 3u) << 4);
-            b.s[g] = scale - 32;
+            b.s[g] = (int)(((head.v[1] >> (4 * g)) & 15u) | ((head.v[0] >> (16 + 2 * g)) & 3u) << 4) - 32;
         }
-        b.d = f16_to_f32(ld16(blk));
+        b.d = f16_to_f32(head.v[0]);
     } else if constexpr (T == kIQ4NL) {
         /* :1129-1175: eight 18-byte blocks */
 #pragma unroll
@@ -294,44 +357,40 @@ __device__ __forceinline__ void decode_lane(const uint8_t *blk, int l, const uin
     } else {
         /* IQ1_S, :1177-1253 */
         const int sec = l >> 1, half = l & 1;
+        const Dwords<4> qh = ldn<4>(blk + 34);
 #pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t high = ld16(blk + 34 + 2 * g);
-            const uint32_t index = blk[2 + 4 * g + sec] | (((high >> (3 * sec)) & 7u) << 8);
-            b.q[g] = iq1s_grid[2 * index + half];
-            b.s[g] = 1 + 2 * (int)((high >> 12) & 7u);
+        for (int p = 0; p < 2; ++p) {
+            const Dwords<4> codes = ldn<4>(blk + 2 + 16 * p);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int g = 4 * p + i;
+                const uint32_t high = (qh.v[g >> 1] >> (16 * (g & 1))) & 0xffffu;
+                const uint32_t index = ((codes.v[i] >> (8 * sec)) & 255u) | (((high >> (3 * sec)) & 7u) << 8);
+                b.q[g] = table[2 * index + half];
+                b.s[g] = 1 + 2 * (int)((high >> 12) & 7u);
+            }
         }
         b.d = f16_to_f32(ld16(blk));
     }
 }
 
-/* the block's integer min (Q2_K, Q5_K) or correction (IQ1_S) term for one
- * token's Q8_K block */
+/* the multipliers of activation sums 2l and 2l + 1 of a block in its integer
+ * min (Q2_K, Q5_K) or correction (IQ1_S) sum */
 template <int T>
-__device__ __forceinline__ int block_extra(const uint8_t *blk, const uint8_t *xb)
+__device__ __forceinline__ void extra_factors(const uint8_t *blk, int l, int &m0, int &m1)
 {
-    const int16_t *sums = reinterpret_cast<const int16_t *>(xb + 260);
-    int extra = 0;
     if constexpr (T == kQ2K) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) extra += (blk[i] >> 4) * sums[i];
-    } else if constexpr (T == kQ5K) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            int sc0, m0, sc1, m1;
-            k4_scale_min(2 * c, blk + 4, sc0, m0);
-            k4_scale_min(2 * c + 1, blk + 4, sc1, m1);
-            extra += m0 * (sums[4 * c] + sums[4 * c + 1]) + m1 * (sums[4 * c + 2] + sums[4 * c + 3]);
-        }
+        const uint32_t w = ld16(blk + 2 * l);
+        m0 = (w >> 4) & 15;
+        m1 = w >> 12;
     } else if constexpr (T == kIQ1S) {
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const uint32_t high = ld16(blk + 34 + 2 * g);
-            const int scale = 1 + 2 * (int)((high >> 12) & 7u);
-            extra += (high & 0x8000u ? -scale : scale) * (sums[2 * g] + sums[2 * g + 1]);
-        }
+        const uint32_t high = ld16(blk + 34 + 2 * l);
+        const int scale = 1 + 2 * (int)((high >> 12) & 7u);
+        m0 = m1 = high & 0x8000u ? -scale : scale;
+    } else {
+        const K4Scales k4 = k4_scales(blk + 4);
+        m0 = m1 = (int)(((l < 4 ? k4.m[0] : k4.m[1]) >> (8 * (l & 3))) & 255u);
     }
-    return extra;
 }
 
 __device__ __forceinline__ float bf16_to_f32(uint32_t bits) { return __uint_as_float(bits << 16); }

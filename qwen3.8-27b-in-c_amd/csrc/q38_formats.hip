@@ -7,11 +7,11 @@
  * 1636-1725) keeps eight fp32 lanes per row; for every super-block, lane l
  * gets d * W[l], where W[l] is the exact integer sum over bytes 4l..4l+3 of
  * each 32-element group, each group-half scaled by its integer sub-block
- * scale.  Here eight GPU lanes own a row's eight accumulator lanes (a
+ * scale.  Here eight GPU lanes stand for a row's eight accumulators (a
  * wavefront holds eight rows): each decodes the four weights of each group
  * it needs into a packed int8 dword (grid value and sign folded in),
- * multiplies with v_dot4_i32_i8 against the activation dword, scales, and
- * runs its fmaf chain.  The eight lanes then add in the reference's tree
+ * multiplies with v_dot4_i32_i8 against the activation dword, scales, and a
+ * wavefront runs the fmaf chains.  The eight lanes then add in the reference's tree
  * ((a0 + a4) + (a2 + a6)) + ((a1 + a5) + (a3 + a7)); Q2_K and Q5_K add their
  * scalar min chain, IQ1_S 0.125 times its scalar correction sum, and IQ4_NL
  * applies one fp32 scale per 32-element group (eight FMAs per block).
@@ -31,69 +31,188 @@ namespace q38 {
 
 namespace {
 
-/* y[t * ldy + row] for t < MT: eight rows per wavefront, eight lanes per row */
+/* Q8_K path for up to eight tokens: y[t * ldy + row].
+ *
+ * A workgroup covers eight rows; its H wavefronts split the blocks,
+ * lane (row r of eight, AVX2 lane l) of each forming the exact integer sums
+ * of its blocks for every token.  The sums (as fp32, exact) and the blocks'
+ * scales go through LDS, and wavefront t runs token t's fp32 chains over the
+ * blocks in order: the integer work of a row is spread over H wavefronts, so
+ * that enough loads are in flight on matrices of few rows, and the order of
+ * the fp32 work stays.  Long rows take several phases of at most kBlocks
+ * blocks.  The IQ codebooks are copied to LDS: a lookup per four weights is
+ * most of these formats' work, and from global memory each costs a cache
+ * access per lane.
+ *
+ * Bound.  Issue of the decode and of the lanes' activation loads.  One token,
+ * 34816 x 5120 / 5120 x 17408: Q5_K 28 / 19 us (4.4 / 3.1 TB/s), Q3_K 31 / 20,
+ * IQ3_S 43 / 29, IQ2_S 54 / 34, IQ1_S 40 / 27 us; eight lanes per row walking
+ * all its blocks took 31 / 51, 32 / 49, 77 / 70, 80 / 72 and 77 / 75 us.
+ * Eight tokens: Q5_K 89 / 58 us (248 / 622 before), IQ3_S 85 / 57 (237 / 499).
+ * H = 8 up to three tokens and 12 for more or for three tokens of long rows:
+ * of 4, 8, 12 and 16 wavefronts Q5_K takes 20 / 19 / 19 / 19 us (one token,
+ * 17408 columns), 84 / 44 / 51 / 76 us (three tokens, 34816 rows), Q3_K 38
+ * (8) and 30 us (12) for three tokens of 17408 columns; 16 or 32 rows per
+ * workgroup measured slower on 5120 rows (25 to 48 us for Q3_K). */
 template <int T, int MT>
-__global__ __launch_bounds__(256) void gemv_format_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ x,
-                                                          float *__restrict__ y, uint32_t ldy, uint32_t rows,
-                                                          uint32_t nb, const uint32_t *__restrict__ iq1s_grid)
-{
-    const int lane = threadIdx.x & 63, l = lane & 7;
-    const uint32_t row = (blockIdx.x * 256u + threadIdx.x) >> 3;
-    const uint32_t r = row < rows ? row : rows - 1;
-    const uint32_t bytes = block_bytes<T>();
-    const uint8_t *wr = w + (size_t)r * nb * bytes;
-    float acc[MT], scalar[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) acc[t] = scalar[t] = 0.0f;
+struct GemvFormat {
+    static constexpr int table = table_dwords<T>() * 4;
+    static constexpr int scalars = T == kIQ1S ? 2 : has_extra<T>() ? 3 : 1;   /* floats per row and block */
+    static constexpr int per_block = MT * (64 + scalars * 8) * 4;
+    static constexpr int kBlocks = (64 * 1024 - table) / per_block;           /* blocks of a phase at most */
+};
 
-    for (uint32_t b = 0; b < nb; ++b) {
-        const uint8_t *blk = wr + (size_t)b * bytes;
-        LaneBlock lb;
-        decode_lane<T>(blk, l, iq1s_grid, lb);
+template <int T, int MT, int H>
+__global__ __launch_bounds__(64 * H) void gemv_format_kernel(const uint8_t *__restrict__ w,
+                                                                const uint8_t *__restrict__ x, float *__restrict__ y,
+                                                                uint32_t ldy, uint32_t rows, uint32_t nb,
+                                                                uint32_t phase_blocks,
+                                                                const uint32_t *__restrict__ iq1s_grid)
+{
+    using F = GemvFormat<T, MT>;
+    constexpr uint32_t kBytes = block_bytes<T>();
+    constexpr int kMine = (MT + H - 1) / H;   /* tokens whose chains a wavefront runs */
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   /* table + phase_blocks * per_block bytes */
+    uint32_t *table = reinterpret_cast<uint32_t *>(lds);
+    /* [block][token][lane], then [block][token][scalar][row] */
+    float *sum_s = reinterpret_cast<float *>(lds + F::table);
+    float *scalar_s = sum_s + phase_blocks * MT * 64;
+    const int lane = threadIdx.x & 63, l = lane & 7, r = lane >> 3;
+    const int h = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const uint32_t row = blockIdx.x * 8 + r;
+    const uint8_t *wr = w + (size_t)(row < rows ? row : rows - 1) * nb * kBytes;
+    if constexpr (F::table > 0) {
+        const uint32_t *src = table_of<T>(iq1s_grid);
+        for (int i = threadIdx.x; i < table_dwords<T>(); i += 64 * H) table[i] = src[i];
+        __syncthreads();
+    }
+    float acc[kMine], scalar[kMine];
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            const uint8_t *xb = x + ((size_t)t * nb + b) * kQ8KBytes;
-            const float xs = *reinterpret_cast<const float *>(xb);
-            const uint32_t *aq = reinterpret_cast<const uint32_t *>(xb + 4);
-            if constexpr (T == kIQ4NL) {
+    for (int i = 0; i < kMine; ++i) acc[i] = scalar[i] = 0.0f;
+
+    for (uint32_t b0 = 0; b0 < nb; b0 += phase_blocks) {
+        const int count = (int)(nb - b0 < phase_blocks ? nb - b0 : phase_blocks);
+        const int first = count * h / H, last = count * (h + 1) / H;
+#pragma unroll 2
+        for (int i = first; i < last; ++i) {
+            const uint32_t b = b0 + i;
+            const uint8_t *blk = wr + (size_t)b * kBytes;
+            LaneBlock lb;
+            decode_lane<T>(blk, l, table, lb);
+            int m0 = 0, m1 = 0;
+            if constexpr (has_extra<T>()) extra_factors<T>(blk, l, m0, m1);
 #pragma unroll
-                for (int g = 0; g < 8; ++g) {
-                    const int wg = dot4z((int)lb.q[g], (int)aq[8 * g + l]);
-                    acc[t] = __builtin_fmaf(__fmul_rn(lb.gd[g], xs), (float)wg, acc[t]);
-                }
-            } else {
+            for (int t = 0; t < MT; ++t) {
+                const uint8_t *xb = x + ((size_t)t * nb + b) * kQ8KBytes;
+                const float xs = *reinterpret_cast<const float *>(xb);
+                const int *aq = reinterpret_cast<const int *>(xb + 4) + l;
+                float *so = sum_s + (size_t)(i * MT + t) * 64 + lane;
+                float *co = scalar_s + (size_t)(i * MT + t) * F::scalars * 8 + r;
                 int wsum = 0;
 #pragma unroll
-                for (int g = 0; g < 8; ++g) wsum += lb.s[g] * dot4z((int)lb.q[g], (int)aq[8 * g + l]);
-                const float d = __fmul_rn(lb.d, xs);
-                acc[t] = __builtin_fmaf(d, (float)wsum, acc[t]);
-                if constexpr (T == kQ2K || T == kQ5K) {
-                    const float dmin = __fmul_rn(lb.dmin, xs);
-                    scalar[t] = __builtin_fmaf(-dmin, (float)block_extra<T>(blk, xb), scalar[t]);
-                } else if constexpr (T == kIQ1S) {
-                    scalar[t] = __fadd_rn(scalar[t], __fmul_rn(d, (float)block_extra<T>(blk, xb)));
+                for (int g = 0; g < 8; ++g) wsum = mad24(lb.s[g], dot4z((int)lb.q[g], aq[8 * g]), wsum);
+                *so = (float)wsum;
+                int extra = 0;
+                if constexpr (has_extra<T>()) {
+                    const int pair = *reinterpret_cast<const int *>(xb + 260 + 4 * l);
+                    extra = quad_sum(m0 * (int)(int16_t)pair + m1 * (pair >> 16));
+                    extra += dpp_move<0x141>(0, extra);   /* the row's other quad */
+                }
+                if (l == 0) {
+                    const float d = fmul_rn(lb.d, xs);
+                    co[0] = d;
+                    if constexpr (T == kIQ1S) {
+                        co[8] = fmul_rn(d, (float)extra);
+                    } else if constexpr (has_extra<T>()) {
+                        co[8] = -fmul_rn(lb.dmin, xs);
+                        co[16] = (float)extra;
+                    }
                 }
             }
         }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kMine; ++k) {
+            const int t = h + k * H;
+            if (t >= MT) break;
+            const float *so = sum_s + (size_t)t * 64 + lane;
+            const float *co = scalar_s + (size_t)t * F::scalars * 8 + r;
+#pragma unroll 4
+            for (int i = 0; i < count; ++i, so += MT * 64, co += MT * F::scalars * 8) {
+                acc[k] = __builtin_fmaf(co[0], so[0], acc[k]);
+                if constexpr (T == kIQ1S) scalar[k] = fadd_rn(scalar[k], co[8]);
+                else if constexpr (has_extra<T>()) scalar[k] = __builtin_fmaf(co[8], co[16], scalar[k]);
+            }
+        }
+        if (b0 + phase_blocks < nb) __syncthreads();
     }
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
+    for (int k = 0; k < kMine; ++k) {
+        const int t = h + k * H;
+        if (t >= MT) break;
         /* ((a0 + a4) + (a2 + a6)) + ((a1 + a5) + (a3 + a7)), qwen38_quant.c:303-310 */
-        float v = __fadd_rn(acc[t], __shfl_xor(acc[t], 4, 64));
-        v = __fadd_rn(v, __shfl_xor(v, 2, 64));
-        v = __fadd_rn(v, __shfl_xor(v, 1, 64));
-        if constexpr (T == kIQ1S) v = __fadd_rn(v, __fmul_rn(0.125f, scalar[t]));
-        else if constexpr (has_extra<T>()) v = __fadd_rn(v, scalar[t]);
+        float v = fadd_rn(acc[k], __shfl_xor(acc[k], 4, 64));
+        v = fadd_rn(v, __shfl_xor(v, 2, 64));
+        v = fadd_rn(v, __shfl_xor(v, 1, 64));
+        if constexpr (T == kIQ1S) v = fadd_rn(v, fmul_rn(0.125f, scalar[k]));
+        else if constexpr (has_extra<T>()) v = fadd_rn(v, scalar[k]);
         if (l == 0 && row < rows) y[(size_t)t * ldy + row] = v;
     }
 }
 
-template <int T, int MT>
+/* IQ4_NL takes one fma per 32-element group instead of one per block, so
+ * handing sums through LDS would cost eight times as much (34816 x 5120, one
+ * token: 83 against 44 us): eight lanes per row, each running its chain over
+ * all blocks. */
+template <int MT>
+__global__ __launch_bounds__(256) void gemv_nl_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ x,
+                                                      float *__restrict__ y, uint32_t ldy, uint32_t rows, uint32_t nb)
+{
+    const int l = threadIdx.x & 7;
+    const uint32_t row = (blockIdx.x * 256u + threadIdx.x) >> 3;
+    const uint8_t *wr = w + (size_t)(row < rows ? row : rows - 1) * nb * block_bytes<kIQ4NL>();
+    float acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[t] = 0.0f;
+    for (uint32_t b = 0; b < nb; ++b) {
+        LaneBlock lb;
+        decode_lane<kIQ4NL>(wr + (size_t)b * block_bytes<kIQ4NL>(), l, nullptr, lb);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const uint8_t *xb = x + ((size_t)t * nb + b) * kQ8KBytes;
+            const float xs = *reinterpret_cast<const float *>(xb);
+            const int *aq = reinterpret_cast<const int *>(xb + 4) + l;
+#pragma unroll
+            for (int g = 0; g < 8; ++g)
+                acc[t] = __builtin_fmaf(fmul_rn(lb.gd[g], xs), (float)dot4z((int)lb.q[g], aq[8 * g]), acc[t]);
+            /* from five tokens on the compiler would move the links past the
+             * other tokens and keep their products in registers (eight tokens,
+             * 34816 x 5120: 353 against 117 us); below, its order is the
+             * faster one (three tokens, 17408 columns: 70 against 113 us) */
+            if constexpr (MT > 4) asm volatile("" : "+v"(acc[t]));
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        float v = fadd_rn(acc[t], __shfl_xor(acc[t], 4, 64));
+        v = fadd_rn(v, __shfl_xor(v, 2, 64));
+        v = fadd_rn(v, __shfl_xor(v, 1, 64));
+        if (l == 0 && row < rows) y[(size_t)t * ldy + row] = v;
+    }
+}
+
+template <int T, int MT, int H>
 void launch_format_typed(const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy, uint32_t rows, uint32_t nb,
                          const void *grid, hipStream_t stream)
 {
-    hipLaunchKernelGGL((gemv_format_kernel<T, MT>), dim3((rows + 31) / 32), dim3(256), 0, stream, w, x, y, ldy, rows,
-                       nb, static_cast<const uint32_t *>(grid));
+    if constexpr (T == kIQ4NL) {
+        hipLaunchKernelGGL(gemv_nl_kernel<MT>, dim3((rows + 31) / 32), dim3(256), 0, stream, w, x, y, ldy, rows, nb);
+        return;
+    }
+    using F = GemvFormat<T, MT>;
+    const uint32_t phases = (nb + F::kBlocks - 1) / F::kBlocks, blocks = (nb + phases - 1) / phases;
+    hipLaunchKernelGGL((gemv_format_kernel<T, MT, H>), dim3((rows + 7) / 8), dim3(64 * H), F::table + blocks * F::per_block,
+                       stream, w, x, y, ldy, rows, nb, blocks, static_cast<const uint32_t *>(grid));
 }
 
 template <int T>
@@ -101,17 +220,19 @@ void launch_format_m(int m, const uint8_t *w, const uint8_t *x, float *y, uint32
                      const void *grid, hipStream_t stream)
 {
     switch (m) {
-    case 1: launch_format_typed<T, 1>(w, x, y, ldy, rows, nb, grid, stream); break;
-    case 2: launch_format_typed<T, 2>(w, x, y, ldy, rows, nb, grid, stream); break;
-    case 3: launch_format_typed<T, 3>(w, x, y, ldy, rows, nb, grid, stream); break;
-    case 4: launch_format_typed<T, 4>(w, x, y, ldy, rows, nb, grid, stream); break;
-    case 5: launch_format_typed<T, 5>(w, x, y, ldy, rows, nb, grid, stream); break;
-    case 6: launch_format_typed<T, 6>(w, x, y, ldy, rows, nb, grid, stream); break;
-    case 7: launch_format_typed<T, 7>(w, x, y, ldy, rows, nb, grid, stream); break;
-    default: launch_format_typed<T, 8>(w, x, y, ldy, rows, nb, grid, stream); break;
+    case 1: launch_format_typed<T, 1, 8>(w, x, y, ldy, rows, nb, grid, stream); break;
+    case 2: launch_format_typed<T, 2, 8>(w, x, y, ldy, rows, nb, grid, stream); break;
+    case 3:
+        if (nb < 40) launch_format_typed<T, 3, 8>(w, x, y, ldy, rows, nb, grid, stream);
+        else launch_format_typed<T, 3, 12>(w, x, y, ldy, rows, nb, grid, stream);
+        break;
+    case 4: launch_format_typed<T, 4, 12>(w, x, y, ldy, rows, nb, grid, stream); break;
+    case 5: launch_format_typed<T, 5, 12>(w, x, y, ldy, rows, nb, grid, stream); break;
+    case 6: launch_format_typed<T, 6, 12>(w, x, y, ldy, rows, nb, grid, stream); break;
+    case 7: launch_format_typed<T, 7, 12>(w, x, y, ldy, rows, nb, grid, stream); break;
+    default: launch_format_typed<T, 8, 12>(w, x, y, ldy, rows, nb, grid, stream); break;
     }
 }
-
 /* ---- row decode ------------------------------------------------------------ */
 
 /* rows[r] of the matrix into out[r * width ..]; the row index of output row

@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kPromptThreads, 1) void gemm_prompt(const uint8_t *
     auto decode = [&]() {
         const uint8_t *blk = lds + L::raw + lane * L::raw_stride;
         LaneBlock lb;
-        decode_lane<T>(blk, wv, iq1s_grid, lb);
+        decode_lane<T>(blk, wv, table_of<T>(iq1s_grid), lb);
         uint8_t *out = lds + L::w0 + 4 * wv * L::wplane + lane * 16;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
@@ -324,19 +324,11 @@ __global__ __launch_bounds__(kPromptThreads, 1) void gemm_prompt(const uint8_t *
                 const int i = wv - 4;   /* the multipliers of sums 4i .. 4i + 3 */
                 half4p m;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    int v;
-                    if constexpr (T == kQ2K) {
-                        v = blk[4 * i + e] >> 4;
-                    } else if constexpr (T == kIQ1S) {
-                        const uint32_t high = ld16(blk + 34 + 2 * (2 * i + e / 2));
-                        v = 1 + 2 * (int)((high >> 12) & 7u);
-                        if (high & 0x8000u) v = -v;
-                    } else {
-                        int sc;
-                        k4_scale_min(2 * i + e / 2, blk + 4, sc, v);
-                    }
-                    m[e] = (_Float16)(float)v;
+                for (int e = 0; e < 2; ++e) {
+                    int m0, m1;
+                    extra_factors<T>(blk, 2 * i + e, m0, m1);
+                    m[2 * e] = (_Float16)(float)m0;
+                    m[2 * e + 1] = (_Float16)(float)m1;
                 }
                 *reinterpret_cast<half4p *>(lds + L::ms + (i * kPromptRows + lane) * 8) = m;
             }
