@@ -3,6 +3,7 @@
  * own for kernel-level parity tests and external callers. */
 #include <hip/hip_runtime.h>
 
+#include <cstring>
 #include <vector>
 
 #include "q38hip.h"
@@ -12,21 +13,23 @@ namespace {
 
 constexpr uint32_t kQGDim = 12288, kQDim = 6144, kKVDim = 1024, kHeads = 24;
 
-struct Buffers {
-    std::vector<void *> owned;
-    ~Buffers()
-    {
-        for (void *p : owned) (void)hipFree(p);
-    }
-    template <typename T>
-    T *get(size_t count)
+/* one device allocation, released at the end of the call */
+struct Workspace {
+    uint8_t *base = nullptr;
+    explicit Workspace(size_t bytes)
     {
         void *p = nullptr;
-        if (hipMalloc(&p, count * sizeof(T)) != hipSuccess) return nullptr;
-        owned.push_back(p);
-        return static_cast<T *>(p);
+        if (hipMalloc(&p, bytes) == hipSuccess) base = static_cast<uint8_t *>(p);
     }
+    ~Workspace()
+    {
+        if (base) (void)hipFree(base);
+    }
+    Workspace(const Workspace &) = delete;
+    Workspace &operator=(const Workspace &) = delete;
 };
+
+constexpr size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 }  // namespace
 
@@ -42,24 +45,38 @@ extern "C" int q38hip_attention_rows(float *attention, Q38Q8KBlock *attention_q8
     if ((uint64_t)position + rows > context_length) return q38::abi_fail("position + rows beyond the context");
     if (context_length > q38::kMaxAttentionContext) return q38::abi_fail("context length above 524256 positions");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    /* drain the caller's earlier work on the stream: the buffers below are
-     * released before return */
-    if (hipStreamSynchronize(s) != hipSuccess) return q38::abi_fail("stream synchronisation failed");
-    Buffers buf;
-    float *rope = buf.get<float>((size_t)context_length * 64);
-    float *q_buf = buf.get<float>((size_t)rows * kQDim);
-    float *scores = buf.get<float>((size_t)rows * kHeads * context_length);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
+        return q38::abi_fail("stream synchronisation failed");
+    /* The host side bounds a call of few rows, so it is kept to one
+     * allocation, one upload and the RoPE rows of the call's own positions
+     * (three rows at a 4K cache: 83 us a call; with the RoPE table of all 5120
+     * positions of the context, five allocations and two uploads 1005 us). */
+    const size_t rope_bytes = align256((size_t)rows * 64 * sizeof(float) + sizeof(uint32_t));
+    const size_t q_bytes = align256((size_t)rows * kQDim * sizeof(float));
+    const size_t score_bytes = align256((size_t)rows * kHeads * context_length * sizeof(float));
+    const size_t out_bytes = attention_q8k ? 0 : (size_t)rows * kHeads * sizeof(Q38Q8KBlock);
+    /* the RoPE rows, then the position word */
+    std::vector<float> table((size_t)rows * 64 + 1);
+    q38::rope_table_host(table.data(), position, rows);
+    std::memcpy(&table[(size_t)rows * 64], &position, sizeof(position));
+    Workspace work(rope_bytes + q_bytes + score_bytes + out_bytes);
+    if (!work.base) return q38::abi_fail("device allocation failed");
+    float *rope = reinterpret_cast<float *>(work.base);
+    uint32_t *pos = reinterpret_cast<uint32_t *>(rope + (size_t)rows * 64);
+    float *q_buf = reinterpret_cast<float *>(work.base + rope_bytes);
+    float *scores = reinterpret_cast<float *>(work.base + rope_bytes + q_bytes);
     uint8_t *q_out = attention_q8k ? reinterpret_cast<uint8_t *>(attention_q8k)
-                                   : buf.get<uint8_t>((size_t)rows * kHeads * sizeof(Q38Q8KBlock));
-    uint32_t *pos = buf.get<uint32_t>(1);
-    if (!rope || !q_buf || !scores || !q_out || !pos) return q38::abi_fail("device allocation failed");
-    std::vector<float> table((size_t)context_length * 64);
-    q38::rope_table_host(table.data(), context_length);
+                                   : work.base + rope_bytes + q_bytes + score_bytes;
     if (hipMemcpyAsync(rope, table.data(), table.size() * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(pos, &position, sizeof(position), hipMemcpyHostToDevice, s) != hipSuccess ||
-        !q38::configure_attention((int)context_length))
+        !q38::configure_attention((int)context_length)) {
+        (void)hipStreamSynchronize(s);
         return q38::abi_fail("attention set-up failed");
-    q38::launch_attention(attention, q_out, q_buf, q_and_gate, key, value, (long long)in_stride, q_norm, k_norm, rope,
+    }
+    /* the kernels index the table by absolute position */
+    const float *rope0 = reinterpret_cast<const float *>(reinterpret_cast<uintptr_t>(rope) -
+                                                         (uintptr_t)position * 64 * sizeof(float));
+    q38::launch_attention(attention, q_out, q_buf, q_and_gate, key, value, (long long)in_stride, q_norm, k_norm, rope0,
                           key_cache, value_cache, scores, (int)context_length, pos, (int)rows, s);
     const hipError_t launched = hipGetLastError();
     const hipError_t done = hipStreamSynchronize(s);

@@ -724,7 +724,7 @@ bool allocate_state(Q38Model *m)
     m->accept = m->words + 32;
     m->sampled = m->words + 48;
     std::vector<float> table((size_t)ctx * 64);
-    q38::rope_table_host(table.data(), ctx);
+    q38::rope_table_host(table.data(), 0, ctx);
     m->query_scale = 1.0f / sqrtf(128.0f);
     return hip_ok(hipMemcpy(m->rope, table.data(), table.size() * sizeof(float), hipMemcpyHostToDevice),
                   "rope table upload");

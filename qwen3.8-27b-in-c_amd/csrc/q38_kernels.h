@@ -184,8 +184,8 @@ void launch_deltanet_out_quant(float *attn, uint8_t *q_out, const float *z, long
 constexpr uint32_t kMaxAttentionContext = 524256;
 __host__ __device__ inline uint32_t value_pitch(uint32_t context) { return (context + 31) & ~31u; }
 bool configure_attention(int context);
-/* host: the RoPE cos/sin table of positions [0, context), 64 floats each */
-void rope_table_host(float *table, uint32_t context);
+/* host: the RoPE cos/sin table of positions first .. first + count - 1, 64 floats each */
+void rope_table_host(float *table, uint32_t first, uint32_t count);
 void launch_attention(float *attn, uint8_t *q_out, float *q_buf, const float *q_and_gate, const float *key,
                       const float *value, long long in_stride, const float *q_norm, const float *k_norm,
                       const float *rope, float *key_cache, float *value_cache, float *scores, int context,

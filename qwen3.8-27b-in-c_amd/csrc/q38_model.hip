@@ -1364,15 +1364,15 @@ bool configure_attention(int context)
     return true;
 }
 
-/* RoPE table of positions [0, context): cos then sin of the 32 pair angles.
+/* RoPE table of positions first .. first + count - 1: cos then sin of the 32 pair angles.
  * theta starts at the position and is multiplied by powf(1e7, -2/64) per
  * pair; cosf/sinf of the host C library, exactly the values q38_rope
  * computes (qwen38_model.c:697-713). */
-void rope_table_host(float *table, uint32_t context)
+void rope_table_host(float *table, uint32_t first, uint32_t count)
 {
     const float theta_scale = powf(10000000.0f, -2.0f / 64.0f);
-    for (uint32_t pos = 0; pos < context; ++pos) {
-        float theta = (float)pos;
+    for (uint32_t pos = 0; pos < count; ++pos) {
+        float theta = (float)(first + pos);
         for (int pair = 0; pair < 32; ++pair) {
             table[(size_t)pos * 64 + pair] = cosf(theta);
             table[(size_t)pos * 64 + 32 + pair] = sinf(theta);
