@@ -49,6 +49,25 @@ def test_random_cases_match_reference(device, checker):
         assert device_sample(case, device) == sc.call(checker, case), case["name"]
 
 
+@pytest.mark.parametrize("top_k", (2, 63, 64, 65))
+def test_selection_edges_match_reference(device, checker, top_k):
+    """around the 1024-logit chunks and 64 candidates of the counting
+    selection: ties across chunks, rows with fewer candidates than top_k and
+    one chunk that holds all of them"""
+    rng = np.random.default_rng(13 + top_k)
+    for vocab in (1023, 1024, 1025, 65537, 70000):
+        noise = rng.standard_normal(vocab).astype(np.float32)
+        peak = noise.copy()
+        peak[:200] += 40.0
+        few = np.full(vocab, -np.inf, np.float32)
+        few[::1 + vocab // 20] = 1.0
+        zeros = np.where(rng.random(vocab) < 0.5, np.float32(0.0), np.float32(-0.0)).astype(np.float32)
+        for name, logits in (("noise", noise), ("ties", np.round(noise)), ("peak", peak), ("few", few), ("zeros", zeros)):
+            case = sc._case(logits, rng.integers(1, 2**63), temperature=0.7, top_k=top_k, top_p=0.97,
+                            name="%s vocab=%d k=%d" % (name, vocab, top_k))
+            assert device_sample(case, device) == sc.call(checker, case), case["name"]
+
+
 def test_state_sequence(device, checker):
     """64 consecutive draws from one row: the state carried from call to
     call as the reference carries it."""
