@@ -223,28 +223,34 @@ __device__ __forceinline__ float avx2_tree16(float a, float b)
  * elements l + 32a and l + 16 + 32a, i.e. P[l] and P[l + 16] as two
  * independent fmaf chains, and avx2_tree16 adds them in the reference's
  * order (measured on MI355X against one column per 32 lanes: 4096-token
- * prefill 422 -> 415 ms).  Sixteen columns of one value head per block of
+ * prefill 422 -> 415 ms).  k and q lie in LDS in a lane's own order, so a
+ * token takes six LDS reads instead of nineteen, and a prompt batch
+ * (LastOnly) has no store or slot arithmetic in the loop: 4096 tokens of one
+ * layer 1.50 -> 1.25 ms, 305 ns a token, of which the two wavefronts of a
+ * SIMD issue about 220.  Two columns per lane row, one wavefront per SIMD,
+ * measured 1.48 ms.  Sixteen columns of one value head per block of
  * 256.  The columns run through `rows` consecutive tokens (row t's prepared
  * q|k|v at qkv + t * ld, beta and alpha at + beta_off / alpha_off, output at
  * out + t * kLinV): the state before row t is slot (*slot_ptr + t), read
  * once, kept in registers, and each row's result is written to the next
- * slot (with `last_only`, only the last row's, to slot *slot_ptr + rows).
+ * slot (with LastOnly, only the last row's, to slot *slot_ptr + rows).
  * The block's inputs (k and q of head h % 16, the block's v values, the
  * decay and beta of head h) come through LDS in chunks of kScanChunk rows,
  * the next chunk's global loads in flight while the current one is
  * scanned, so the sequential scan reads only LDS. */
 constexpr int kScan16Cols = 16;
 
+template <bool LastOnly>
 __global__ __launch_bounds__(256) void deltanet_state_kernel(float *__restrict__ out, float *__restrict__ state,
                                                               long long slot_stride,
                                                               const uint32_t *__restrict__ slot_ptr, int rows,
                                                               const float *__restrict__ qkv, long long ld,
-                                                              int beta_off, int alpha_off, float query_scale,
-                                                              int last_only)
+                                                              int beta_off, int alpha_off, float query_scale)
 {
-    __shared__ float kq_s[2][kScanChunk][2 * kHeadDim];   /* [parity][row][k 0..127 | q 0..127] */
+    /* [parity][row][k | q][half][lane][4]: lane l's elements 32a + l and 32a + 16 + l */
+    __shared__ __attribute__((aligned(16))) float kq_s[2][kScanChunk][2 * kHeadDim];
     __shared__ float v_s[2][kScanChunk][kScan16Cols];
-    __shared__ float ab_s[2][kScanChunk][2];               /* decay = expf(alpha), beta */
+    __shared__ __attribute__((aligned(8))) float ab_s[2][kScanChunk][2];   /* decay = expf(alpha), beta */
     const int tid = threadIdx.x;
     const int col0 = blockIdx.x * kScan16Cols;   /* 0 .. 48*128-1 */
     const int h = col0 >> 7;
@@ -266,6 +272,7 @@ __global__ __launch_bounds__(256) void deltanet_state_kernel(float *__restrict__
      * chunk, the v value of row tid / 16 and column tid % 16, and threads
      * 0..2R-1 an alpha or beta */
     const int kq_src = tid < kHeadDim ? kQKDim + kh * kHeadDim + tid : kh * kHeadDim + (tid - kHeadDim);
+    const int kq_dst = (tid & 128) + ((tid & 16) << 2) + ((tid & 15) << 2) + ((tid >> 5) & 3);
     float kq_r[kScanChunk], v_r = 0.0f, ab_r = 0.0f;
     const int nchunks = (rows + kScanChunk - 1) / kScanChunk;
     auto fetch = [&](int ch) {
@@ -288,7 +295,7 @@ __global__ __launch_bounds__(256) void deltanet_state_kernel(float *__restrict__
     };
     auto stage = [&](int par) {
 #pragma unroll
-        for (int i = 0; i < kScanChunk; ++i) kq_s[par][i][tid] = kq_r[i];
+        for (int i = 0; i < kScanChunk; ++i) kq_s[par][i][kq_dst] = kq_r[i];
         v_s[par][tid >> 4][tid & 15] = v_r;
         if (tid < 2 * kScanChunk) ab_s[par][tid >> 1][tid & 1] = (tid & 1) ? ab_r : q38_expf(ab_r);
     };
@@ -298,16 +305,31 @@ __global__ __launch_bounds__(256) void deltanet_state_kernel(float *__restrict__
     auto read_row = [&](int par, int i) {
         RowIn in;
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            in.k[a] = kq_s[par][i][32 * a + l];
-            in.k[4 + a] = kq_s[par][i][32 * a + l + 16];
-            in.q[a] = kq_s[par][i][kHeadDim + 32 * a + l];
-            in.q[4 + a] = kq_s[par][i][kHeadDim + 32 * a + l + 16];
+        for (int half = 0; half < 2; ++half) {
+            const float4 kk = *reinterpret_cast<const float4 *>(&kq_s[par][i][64 * half + 4 * l]);
+            const float4 qq = *reinterpret_cast<const float4 *>(&kq_s[par][i][kHeadDim + 64 * half + 4 * l]);
+            in.k[4 * half] = kk.x;
+            in.k[4 * half + 1] = kk.y;
+            in.k[4 * half + 2] = kk.z;
+            in.k[4 * half + 3] = kk.w;
+            in.q[4 * half] = qq.x;
+            in.q[4 * half + 1] = qq.y;
+            in.q[4 * half + 2] = qq.z;
+            in.q[4 * half + 3] = qq.w;
         }
         in.v = v_s[par][i][cl];
-        in.beta = ab_s[par][i][1];
-        in.decay = ab_s[par][i][0];
+        const float2 ab = *reinterpret_cast<const float2 *>(ab_s[par][i]);
+        in.beta = ab.y;
+        in.decay = ab.x;
         return in;
+    };
+    auto write_state = [&](int t) {
+        float *s_out = state + (size_t)((slot0 + t + 1) % kStateSlots) * slot_stride + col_off;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            s_out[32 * a + l] = sv[a];
+            s_out[32 * a + l + 16] = sv[4 + a];
+        }
     };
     fetch(0);
     stage(0);
@@ -331,27 +353,23 @@ __global__ __launch_bounds__(256) void deltanet_state_kernel(float *__restrict__
             }
             const float pred = avx2_tree16(pa, pb);
             const float delta = __fmul_rn(__fsub_rn(cur.v, pred), cur.beta);
-            float *s_out = state + (size_t)((slot0 + t + 1) % kStateSlots) * slot_stride + col_off;
-            const bool store = !last_only || t == rows - 1;
             float ra = 0.0f, rb = 0.0f;
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
                 sv[a] = __builtin_fmaf(cur.k[a], delta, sv[a]);
                 sv[4 + a] = __builtin_fmaf(cur.k[4 + a], delta, sv[4 + a]);
-                if (store) {
-                    s_out[32 * a + l] = sv[a];
-                    s_out[32 * a + l + 16] = sv[4 + a];
-                }
                 ra = __builtin_fmaf(sv[a], cur.q[a], ra);
                 rb = __builtin_fmaf(sv[4 + a], cur.q[4 + a], rb);
             }
             const float result = avx2_tree16(ra, rb);
             if (l == 0) out[(size_t)t * kLinV + h * kHeadDim + c] = __fmul_rn(result, query_scale);
+            if (!LastOnly) write_state(t);
             cur = nxt;
         }
         if (ch + 1 < nchunks) stage(par ^ 1);
         __syncthreads();
     }
+    if (LastOnly) write_state(rows - 1);
 }
 
 /* Prefill form of deltanet_prep_kernel.  The conv of row t reads only the
@@ -1320,8 +1338,13 @@ void launch_deltanet_state(float *attn, float *delta_state, long long slot_strid
                            const float *qkv, long long ld, int beta_off, int alpha_off, float query_scale,
                            bool last_only, hipStream_t stream)
 {
-    deltanet_state_kernel<<<kVHeads * kHeadDim / kScan16Cols, 256, 0, stream>>>(
-        attn, delta_state, slot_stride, slot, rows, qkv, ld, beta_off, alpha_off, query_scale, last_only ? 1 : 0);
+    const dim3 grid(kVHeads * kHeadDim / kScan16Cols);
+    if (last_only)
+        deltanet_state_kernel<true><<<grid, 256, 0, stream>>>(attn, delta_state, slot_stride, slot, rows, qkv, ld,
+                                                             beta_off, alpha_off, query_scale);
+    else
+        deltanet_state_kernel<false><<<grid, 256, 0, stream>>>(attn, delta_state, slot_stride, slot, rows, qkv, ld,
+                                                              beta_off, alpha_off, query_scale);
 }
 
 bool launch_deltanet_fused(float *attn, float *delta_state, long long slot_stride, const uint32_t *slot, int rows,
