@@ -56,7 +56,10 @@ bool launch_gemm_q4k_mm16(int m, const uint8_t *w_tiled, const uint8_t *x, float
  * launch_gemm_q4k_tiled takes it from kWideMinTokens tokens on. */
 constexpr int kWideMinTokens = 9;
 bool launch_gemm_q4k_wide(uint32_t tokens, const uint8_t *w_tiled, const uint8_t *x, float *y, uint32_t ldy,
-                          uint32_t rows, uint32_t nb, hipStream_t stream);
+                          uint32_t rows, uint32_t nb, hipStream_t stream, void *operands = nullptr);
+/* bytes of the workspace `operands`, with which the activations are converted
+ * once, ahead of the product (16-byte aligned; one call at a time uses it) */
+size_t wide_operand_bytes(uint32_t tokens, uint32_t nb);
 /* same with the token rows of y `ldy` floats apart (ldy >= rows) */
 bool launch_gemm_ld(int type, int m, const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy, uint32_t rows,
                     uint32_t nblk, const void *grid, hipStream_t stream);

@@ -33,6 +33,15 @@
  * it owns.  The two lane halves of a (row, token) meet in LDS for the final
  * tree.  Activation scales and sub-block pair sums of the workgroup's 64
  * tokens are staged in LDS once.
+ *
+ * Bound.  Vector issue: 341 instructions per wavefront and block when it
+ * converts its own activations, 245 with the operands prepared by
+ * wide_operands_kernel (7 us per 512 x 5120 batch), against 384 cycles of
+ * matrix cores.  512 tokens: 34816 x 5120 611 -> 519 us (352 TFLOP/s), 5120 x
+ * 17408 334 -> 274, 16480 x 5120 325 -> 273, 5120 x 6144 127 -> 105 us.  The
+ * engine keeps the operand buffer; callers without a workspace (the C ABI's
+ * one-call GEMM) take the converting form, since the buffer would have to be
+ * allocated on each call.
  */
 #include "q38_device.h"
 #include "q38_kernels.h"
@@ -46,12 +55,34 @@ typedef float float16v_w __attribute__((ext_vector_type(16)));
 
 constexpr int kWideRows = 64, kWideTokens = 64, kWideWaves = 8;
 
-/* loads of one block for one lane */
+/* weight loads of one block for one lane */
 struct WideBlk {
     uint4 h;          /* header of the lane's row: d|dmin, 12 scale/min bytes */
     uint4 wq[2];      /* quant dwords 4 lh .. 4 lh + 3 of chunks q and q + 2 */
-    uint4 lo[2], hi[2];   /* activation dwords 4 lh .. of chunks q, q + 2: low and high halves */
 };
+/* activation operands of one block for one lane: fp16 products' A inputs of
+ * AVX2 lanes 4 lh + k, chunks q (a0) and q + 2 (a1) */
+struct WideAct {
+    half8 a0[4], a1[4];
+};
+
+/* int8 activations as the fp16 operands above, one 16-byte unit per (block,
+ * chunk, AVX2 lane, token), tokens consecutive and padded with zeros to
+ * `padded`: the kernel's loads are then whole cache lines, and each
+ * activation is converted once instead of once per 32 weight rows */
+__global__ __launch_bounds__(256) void wide_operands_kernel(const uint8_t *__restrict__ x, uint4 *__restrict__ out,
+                                                            uint32_t nb, uint32_t tokens, uint32_t padded)
+{
+    const uint32_t unit = blockIdx.y, b = unit >> 5, c = (unit >> 3) & 3, l = unit & 7;
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    if (t >= padded) return;
+    half8 v = {};
+    if (t < tokens) {
+        const uint8_t *q = x + ((size_t)t * nb + b) * kQ8KBytes + 4 + 64 * c + 4 * l;
+        v = act8(*reinterpret_cast<const uint32_t *>(q), *reinterpret_cast<const uint32_t *>(q + 32));
+    }
+    out[(size_t)unit * padded + t] = __builtin_bit_cast(uint4, v);
+}
 
 /* LDS: the staged scales (fp32) and pair sums (8 x int16) of the tile's
  * tokens, later reused for the final exchange (four wavefronts x eight
@@ -68,9 +99,12 @@ constexpr int wide_lds_bytes()
     return wide_stage_bytes<NB>() > kWideExchangeBytes ? wide_stage_bytes<NB>() : kWideExchangeBytes;
 }
 
-template <int NB>
+/* Operands: activations come from wide_operands_kernel's planes xh (tokens
+ * padded to `padded`), else the kernel converts the Q8_K quants itself */
+template <int NB, bool Operands>
 __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_t *__restrict__ w,
                                                                    const uint8_t *__restrict__ x,
+                                                                   const uint4 *__restrict__ xh, uint32_t padded,
                                                                    float *__restrict__ y, uint32_t ldy,
                                                                    uint32_t rows, uint32_t tokens)
 {
@@ -122,7 +156,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_
 
     auto load = [&](int b) {
         const int bb = b < NB ? b : NB - 1;   /* past the end: re-read the last block, unused */
-        const int wo = bb * kTileBlock, xo = bb * kQ8KBytes;
+        const int wo = bb * kTileBlock;
         WideBlk c;
         int4v v = __builtin_amdgcn_raw_buffer_load_b128(wr, hoff, wo, 0);
         c.h = make_uint4(v[0], v[1], v[2], v[3]);
@@ -130,14 +164,44 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_
         c.wq[0] = make_uint4(v[0], v[1], v[2], v[3]);
         v = __builtin_amdgcn_raw_buffer_load_b128(wr, woff1, wo, 0);
         c.wq[1] = make_uint4(v[0], v[1], v[2], v[3]);
-        v = __builtin_amdgcn_raw_buffer_load_b128(xr, xoff0, xo, 0);
-        c.lo[0] = make_uint4(v[0], v[1], v[2], v[3]);
-        v = __builtin_amdgcn_raw_buffer_load_b128(xr, xoff0 + 32, xo, 0);
-        c.hi[0] = make_uint4(v[0], v[1], v[2], v[3]);
-        v = __builtin_amdgcn_raw_buffer_load_b128(xr, xoff1, xo, 0);
-        c.lo[1] = make_uint4(v[0], v[1], v[2], v[3]);
-        v = __builtin_amdgcn_raw_buffer_load_b128(xr, xoff1 + 32, xo, 0);
-        c.hi[1] = make_uint4(v[0], v[1], v[2], v[3]);
+        return c;
+    };
+    /* converted operands: unit (32 b + 8 chunk + lane) * padded + token */
+    const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint4 *>(xh), 0, Operands ? (uint32_t)NB * 32u * padded * 16u : 0u, kRawBuffer);
+    const uint32_t ho = ((uint32_t)(8 * q + 4 * lh) * padded + tok0 + atok) * 16u;
+    auto load_half = [&](int b, int chunk, int k) {
+        const int bb = b < NB ? b : NB - 1;
+        const uint32_t so = (uint32_t)(32 * bb + 8 * chunk + k) * padded * 16u;
+        return __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(hr, ho, so, 0));
+    };
+    auto load_act = [&](int b) {
+        WideAct a;
+        if constexpr (Operands) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                a.a0[k] = load_half(b, 0, k);
+                a.a1[k] = load_half(b, 2, k);
+            }
+        }
+        return a;
+    };
+    struct RawAct {
+        uint4 lo[2], hi[2];   /* activation dwords 4 lh .. of chunks q, q + 2: low and high halves */
+    };
+    auto load_raw = [&](int b) {
+        RawAct c = {};
+        if constexpr (!Operands) {
+            const int xo = (b < NB ? b : NB - 1) * kQ8KBytes;
+            int4v v = __builtin_amdgcn_raw_buffer_load_b128(xr, xoff0, xo, 0);
+            c.lo[0] = make_uint4(v[0], v[1], v[2], v[3]);
+            v = __builtin_amdgcn_raw_buffer_load_b128(xr, xoff0 + 32, xo, 0);
+            c.hi[0] = make_uint4(v[0], v[1], v[2], v[3]);
+            v = __builtin_amdgcn_raw_buffer_load_b128(xr, xoff1, xo, 0);
+            c.lo[1] = make_uint4(v[0], v[1], v[2], v[3]);
+            v = __builtin_amdgcn_raw_buffer_load_b128(xr, xoff1 + 32, xo, 0);
+            c.hi[1] = make_uint4(v[0], v[1], v[2], v[3]);
+        }
         return c;
     };
 
@@ -155,9 +219,12 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_
     const int dtok = 32 * tt + 4 * q;
 
     WideBlk cur = load(0);
+    WideAct act = load_act(0);
+    RawAct raw = load_raw(0);
 #pragma unroll 1
     for (int b = 0; b < NB; ++b) {
         const WideBlk nxt = load(b + 1);
+        const RawAct raw_nxt = load_raw(b + 1);
         /* 6-bit scales of chunks q and q + 2 (qwen38_quant.c:131-143) */
         const uint32_t Y = cur.h.y, Z = cur.h.z, Wd = cur.h.w;
         const uint32_t scw[2] = {Y & 0x3f3f3f3fu, (Wd & 0x0f0f0f0fu) | ((Y >> 2) & 0x30303030u)};
@@ -195,22 +262,28 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_
         for (int j = 0; j < 16; ++j) dx[j] = fmul_rn(dh, xsv[j]);
         const uint32_t wq0[4] = {cur.wq[0].x, cur.wq[0].y, cur.wq[0].z, cur.wq[0].w};
         const uint32_t wq1[4] = {cur.wq[1].x, cur.wq[1].y, cur.wq[1].z, cur.wq[1].w};
-        const uint32_t lo0[4] = {cur.lo[0].x, cur.lo[0].y, cur.lo[0].z, cur.lo[0].w};
-        const uint32_t hi0[4] = {cur.hi[0].x, cur.hi[0].y, cur.hi[0].z, cur.hi[0].w};
-        const uint32_t lo1[4] = {cur.lo[1].x, cur.lo[1].y, cur.lo[1].z, cur.lo[1].w};
-        const uint32_t hi1[4] = {cur.hi[1].x, cur.hi[1].y, cur.hi[1].z, cur.hi[1].w};
+        const uint32_t lo0[4] = {raw.lo[0].x, raw.lo[0].y, raw.lo[0].z, raw.lo[0].w};
+        const uint32_t hi0[4] = {raw.hi[0].x, raw.hi[0].y, raw.hi[0].z, raw.hi[0].w};
+        const uint32_t lo1[4] = {raw.lo[1].x, raw.lo[1].y, raw.lo[1].z, raw.lo[1].w};
+        const uint32_t hi1[4] = {raw.hi[1].x, raw.hi[1].y, raw.hi[1].z, raw.hi[1].w};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const half8 b0 = dequant(wq0[k], sc[0], kMask, kMaskHi, kMagic);
             const half8 b1 = dequant(wq1[k], sc[1], kMask, kMaskHi, kMagic);
-            const half8 a0 = act8(lo0[k], hi0[k]);
-            const half8 a1 = act8(lo1[k], hi1[k]);
+            const half8 a0 = Operands ? act.a0[k] : act8(lo0[k], hi0[k]);
+            const half8 a1 = Operands ? act.a1[k] : act8(lo1[k], hi1[k]);
             float16v_w d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b0, z, 0, 0, 0);
             d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b1, d, 0, 0, 0);
+            if constexpr (Operands) {
+                /* the next block's operand into the registers just read */
+                act.a0[k] = load_half(b + 1, 0, k);
+                act.a1[k] = load_half(b + 1, 2, k);
+            }
 #pragma unroll
             for (int j = 0; j < 16; ++j) acc[j][k] = __builtin_fmaf(dx[j], d[j], acc[j][k]);
         }
         cur = nxt;
+        raw = raw_nxt;
     }
 
     /* final tree: the lane half lh = 1 hands its six values per (row, token)
@@ -251,29 +324,48 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_
     }
 }
 
-template <int NB>
-bool launch_wide_nb(const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy, uint32_t rows, uint32_t tokens,
-                    hipStream_t stream)
+template <int NB, bool Operands>
+bool launch_wide_nb(const uint8_t *w, const uint8_t *x, const uint4 *xh, uint32_t padded, float *y, uint32_t ldy,
+                    uint32_t rows, uint32_t tokens, hipStream_t stream)
 {
     static_assert(wide_lds_bytes<NB>() <= 160 * 1024, "LDS");
-    hipLaunchKernelGGL(gemm_q4k_wide<NB>, dim3((rows + kWideRows - 1) / kWideRows, (tokens + kWideTokens - 1) / kWideTokens),
-                       dim3(64 * kWideWaves), 0, stream, w, x, y, ldy, rows, tokens);
+    hipLaunchKernelGGL((gemm_q4k_wide<NB, Operands>),
+                       dim3((rows + kWideRows - 1) / kWideRows, (tokens + kWideTokens - 1) / kWideTokens),
+                       dim3(64 * kWideWaves), 0, stream, w, x, xh, padded, y, ldy, rows, tokens);
     return hipGetLastError() == hipSuccess;
 }
 
-}  // namespace
-
-bool launch_gemm_q4k_wide(uint32_t tokens, const uint8_t *w_tiled, const uint8_t *x, float *y, uint32_t ldy,
-                          uint32_t rows, uint32_t nb, hipStream_t stream)
+template <bool Operands>
+bool launch_wide(uint32_t tokens, const uint8_t *w, const uint8_t *x, const uint4 *xh, uint32_t padded, float *y,
+                 uint32_t ldy, uint32_t rows, uint32_t nb, hipStream_t stream)
 {
-    if (!rows || !tokens || ldy < rows || tokens > 65535u * kWideTokens) return false;
     switch (nb) {
-    case 20: return launch_wide_nb<20>(w_tiled, x, y, ldy, rows, tokens, stream);
-    case 24: return launch_wide_nb<24>(w_tiled, x, y, ldy, rows, tokens, stream);
-    case 40: return launch_wide_nb<40>(w_tiled, x, y, ldy, rows, tokens, stream);
-    case 68: return launch_wide_nb<68>(w_tiled, x, y, ldy, rows, tokens, stream);
+    case 20: return launch_wide_nb<20, Operands>(w, x, xh, padded, y, ldy, rows, tokens, stream);
+    case 24: return launch_wide_nb<24, Operands>(w, x, xh, padded, y, ldy, rows, tokens, stream);
+    case 40: return launch_wide_nb<40, Operands>(w, x, xh, padded, y, ldy, rows, tokens, stream);
+    case 68: return launch_wide_nb<68, Operands>(w, x, xh, padded, y, ldy, rows, tokens, stream);
     default: return false;
     }
+}
+
+uint32_t padded_tokens(uint32_t tokens) { return (tokens + kWideTokens - 1) / kWideTokens * kWideTokens; }
+
+}  // namespace
+
+size_t wide_operand_bytes(uint32_t tokens, uint32_t nb) { return (size_t)nb * 32 * padded_tokens(tokens) * 16; }
+
+bool launch_gemm_q4k_wide(uint32_t tokens, const uint8_t *w_tiled, const uint8_t *x, float *y, uint32_t ldy,
+                          uint32_t rows, uint32_t nb, hipStream_t stream, void *operands)
+{
+    if (!rows || !tokens || ldy < rows || tokens > 65535u * kWideTokens) return false;
+    if (nb != 20 && nb != 24 && nb != 40 && nb != 68) return false;
+    if (!operands || wide_operand_bytes(tokens, nb) > 0xffffffffull)
+        return launch_wide<false>(tokens, w_tiled, x, nullptr, 0, y, ldy, rows, nb, stream);
+    const uint32_t padded = padded_tokens(tokens);
+    uint4 *xh = static_cast<uint4 *>(operands);
+    hipLaunchKernelGGL(wide_operands_kernel, dim3((padded + 255) / 256, nb * 32), dim3(256), 0, stream, x, xh, nb, tokens,
+                       padded);
+    return launch_wide<true>(tokens, w_tiled, x, xh, padded, y, ldy, rows, nb, stream);
 }
 
 }  // namespace q38
