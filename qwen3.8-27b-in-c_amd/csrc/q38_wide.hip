@@ -20,8 +20,9 @@
  * and int8 activations are exact in fp16, every partial sum is an integer
  * below 2^24): two v_mfma_f32_32x32x16_f16 per lane l, A = 32 tokens,
  * B = 32 weight rows, with no redundant products.  The min sums are
- * v_mfma_f32_32x32x2_f32 with K = the two sub-blocks of a chunk (products
- * below 2^19, exact).
+ * v_mfma_f32_32x32x8_f16 over the two sub-blocks of a chunk, each int16 pair
+ * sum split into a multiple of 64 and a rest (both exact in fp16, products
+ * below 2^21): half the matrix-core time of the fp32 product.
  *
  * Layout.  A workgroup of 8 wavefronts covers 64 rows x 64 tokens.
  * Wavefront w: lane half lh = w & 1 (AVX2 lanes 4 lh .. 4 lh + 3, min lanes
@@ -35,10 +36,13 @@
  * tokens are staged in LDS once.
  *
  * Bound.  Vector issue: 341 instructions per wavefront and block when it
- * converts its own activations, 245 with the operands prepared by
- * wide_operands_kernel (7 us per 512 x 5120 batch), against 384 cycles of
- * matrix cores.  512 tokens: 34816 x 5120 611 -> 519 us (352 TFLOP/s), 5120 x
- * 17408 334 -> 274, 16480 x 5120 325 -> 273, 5120 x 6144 127 -> 105 us.  The
+ * converts its own activations, 247 with the operands prepared by
+ * wide_operands_kernel (7 us per 512 x 5120 batch), against 320 cycles of
+ * matrix cores (384 with fp32 min products).  512 tokens, converting with
+ * fp32 min products / prepared operands / those and fp16 min products:
+ * 34816 x 5120 611 / 519 / 489 us (373 TFLOP/s), 5120 x 17408 334 / 274 / 257,
+ * 16480 x 5120 325 / 273 / 258, 5120 x 6144 127 / 105 / 99 us; converting with
+ * fp16 min products 585 us (34816 x 5120) and 311 us (5120 x 17408).  The
  * engine keeps the operand buffer; callers without a workspace (the C ABI's
  * one-call GEMM) take the converting form, since the buffer would have to be
  * allocated on each call.
@@ -52,6 +56,7 @@ namespace q38 {
 namespace {
 
 typedef float float16v_w __attribute__((ext_vector_type(16)));
+typedef _Float16 half4w __attribute__((ext_vector_type(4)));
 
 constexpr int kWideRows = 64, kWideTokens = 64, kWideWaves = 8;
 
@@ -84,13 +89,13 @@ __global__ __launch_bounds__(256) void wide_operands_kernel(const uint8_t *__res
     out[(size_t)unit * padded + t] = __builtin_bit_cast(uint4, v);
 }
 
-/* LDS: the staged scales (fp32) and pair sums (8 x int16) of the tile's
+/* LDS: the staged scales (fp32) and pair sums (8 x two fp16) of the tile's
  * tokens, later reused for the final exchange (four wavefronts x eight
  * tokens x six values x 64 lanes) */
 template <int NB>
 constexpr int wide_stage_bytes()
 {
-    return NB * kWideTokens * (4 + 16);
+    return NB * kWideTokens * (4 + 32);
 }
 constexpr int kWideExchangeBytes = 4 * 8 * 6 * 64 * 4;
 template <int NB>
@@ -108,10 +113,11 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_
                                                                    float *__restrict__ y, uint32_t ldy,
                                                                    uint32_t rows, uint32_t tokens)
 {
-    /* xs_s[b][t]: activation scale; ps_s[b][t][j]: pair sums s[2j] + s[2j+1] */
+    /* xs_s[b][t]: activation scale; ps_s[b][t][j]: the int16 pair sum
+     * s[2j] + s[2j+1] as fp16, its multiple of 64 and the rest */
     __shared__ __attribute__((aligned(16))) uint8_t lds[wide_lds_bytes<NB>()];
     float *xs_s = reinterpret_cast<float *>(lds);
-    int16_t *ps_s = reinterpret_cast<int16_t *>(lds + NB * kWideTokens * 4);
+    half2v *ps_s = reinterpret_cast<half2v *>(lds + NB * kWideTokens * 4);
 
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -145,11 +151,15 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_
         const int4v s0 = __builtin_amdgcn_raw_buffer_load_b128(xr, base + 260, 0, 0);
         const int4v s1 = __builtin_amdgcn_raw_buffer_load_b128(xr, base + 276, 0, 0);
         xs_s[i] = __uint_as_float(sc);
-        int16_t *ps = ps_s + (size_t)i * 8;
+        half2v *ps = ps_s + (size_t)i * 8;
+        auto split = [](int v) {
+            const int sum = (int16_t)((int)(int16_t)(v & 0xffff) + (v >> 16));
+            return (half2v){(_Float16)(float)(sum & ~63), (_Float16)(float)(sum & 63)};
+        };
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            ps[k] = (int16_t)((int)(int16_t)(s0[k] & 0xffff) + (s0[k] >> 16));
-            ps[4 + k] = (int16_t)((int)(int16_t)(s1[k] & 0xffff) + (s1[k] >> 16));
+            ps[k] = split(s0[k]);
+            ps[4 + k] = split(s1[k]);
         }
     }
     __syncthreads();
@@ -215,6 +225,14 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_
     uint32_t kMask = 0x000f000fu, kMaskHi = 0x00f000f0u, kMagic = 0x64006400u;
     asm volatile("" : "+v"(kMask), "+v"(kMaskHi), "+v"(kMagic));
     const uint32_t sel_lo = 0x07000700u + (uint32_t)(2 * q) * 0x00010001u;
+    const uint32_t sel_min = 0x07000700u + (uint32_t)q * 0x00010001u;
+    /* one min lane's two sub-blocks (one per lane half): (high, rest) of the
+     * pair sum times (m, m), the other two K-slots zero */
+    auto min_product = [](half2v sums, half2v m) {
+        const float16v_w none = {};
+        return __builtin_amdgcn_mfma_f32_32x32x8f16((half4w){sums[0], sums[1], 0, 0}, (half4w){m[0], m[1], 0, 0}, none, 0,
+                                                    0, 0);
+    };
     /* LDS index of the lane's D tokens: 32 tt + 8 (j / 4) + 4 q + j % 4 */
     const int dtok = 32 * tt + 4 * q;
 
@@ -239,10 +257,10 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_
         }
         /* mins of sub-blocks 4 lh + q and 4 lh + 2 + q (bytes q, 2 + q) */
         const uint32_t mw = lh ? (((Wd >> 4) & 0x0f0f0f0fu) | ((Z >> 2) & 0x30303030u)) : (Z & 0x3f3f3f3fu);
-        const float mn0 = (float)((mw >> (8 * q)) & 63u), mn1 = (float)((mw >> (8 * q + 16)) & 63u);
+        const half2v mn0 = pair_byte(mw, sel_min), mn1 = pair_byte(mw, sel_min + 0x00020002u);
         /* pair sums of the A token for the two min products */
-        const int16_t *ps = ps_s + ((size_t)b * kWideTokens + atok) * 8;
-        const float pa0 = (float)ps[4 * lh + q], pa1 = (float)ps[4 * lh + 2 + q];
+        const half2v *ps = ps_s + ((size_t)b * kWideTokens + atok) * 8 + 4 * lh + q;
+        const half2v pa0 = ps[0], pa1 = ps[2];
         const float16v_w z = {};
         const float dh = f16_to_f32(cur.h.x), dmh = f16_to_f32(cur.h.x >> 16);
         const float *xsb = xs_s + b * kWideTokens + dtok;
@@ -250,10 +268,10 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void gemm_q4k_wide(const uint8_
 #pragma unroll
         for (int j = 0; j < 16; ++j) xsv[j] = xsb[8 * (j >> 2) + (j & 3)];
         {
-            const float16v_w m0 = __builtin_amdgcn_mfma_f32_32x32x2f32(pa0, mn0, z, 0, 0, 0);
+            const float16v_w m0 = min_product(pa0, mn0);
 #pragma unroll
             for (int j = 0; j < 16; ++j) accm[j][0] = __builtin_fmaf(-fmul_rn(dmh, xsv[j]), m0[j], accm[j][0]);
-            const float16v_w m1 = __builtin_amdgcn_mfma_f32_32x32x2f32(pa1, mn1, z, 0, 0, 0);
+            const float16v_w m1 = min_product(pa1, mn1);
 #pragma unroll
             for (int j = 0; j < 16; ++j) accm[j][1] = __builtin_fmaf(-fmul_rn(dmh, xsv[j]), m1[j], accm[j][1]);
         }
