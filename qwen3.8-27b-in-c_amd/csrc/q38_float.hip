@@ -84,7 +84,7 @@ struct QuadLoad<kF32> {
     __device__ __forceinline__ void load(const uint8_t *row, uint32_t c, uint32_t width)
     {
         const uint8_t *p = row + 4 * (size_t)c;
-        if (!Edge || c + 4 <= width) __builtin_memcpy(v, p, 16);
+        if (!Edge || c + 3 < width) __builtin_memcpy(v, p, 16);
         else
             for (int k = 0; k < 4; ++k) v[k] = c + k < width ? *reinterpret_cast<const float *>(p + 4 * k) : 0.0f;
     }
@@ -100,7 +100,7 @@ struct QuadLoad16 {
     __device__ __forceinline__ void load(const uint8_t *row, uint32_t c, uint32_t width)
     {
         const uint8_t *p = row + 2 * (size_t)c;
-        if (!Edge || c + 4 <= width) {
+        if (!Edge || c + 3 < width) {
             __builtin_memcpy(v, p, 8);
         } else {
             uint32_t h[4];
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(64 * CW + kProducers, ST == 128 ? 2 : CW == 1 ? 5 :
                 const int t = (tid + k * kProducers) / kFloatQuads;
                 const uint32_t tok = tok0 + (t < kTok ? t : kTok - 1);
                 const float *xr = x + (size_t)(tok < tokens ? tok : tokens - 1) * width;
-                if (chain_column<T>(1) == 1 && (!Edge || c + 4 <= width)) {
+                if (chain_column<T>(1) == 1 && (!Edge || c + 3 < width)) {
                     __builtin_memcpy(&s.x[k], xr + c, 16);
                 } else {
                     float v[4];
@@ -431,14 +431,11 @@ bool launch_float_t(const uint8_t *w, const float *x, float *y, uint32_t ldy, ui
 
 }  // namespace
 
-bool launch_gemm_float(int type, uint32_t m, const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows,
-                       uint32_t width, hipStream_t stream)
+namespace {
+
+bool launch_float_rows(int type, uint32_t m, const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows,
+                       uint32_t width, uint32_t row_bytes, hipStream_t stream)
 {
-    uint32_t e = 0, b = 0;
-    if (m < 1 || ldy < rows || !rows || !width || !format_block_shape(type, &e, &b) || width % e ||
-        m > 65535u * 64 || (uint64_t)width / e * b * kFloatRows > 0xffffffffull)
-        return false;   /* the workgroup's rows are addressed with 32-bit offsets */
-    const uint32_t row_bytes = (uint32_t)((uint64_t)width / e * b);
     switch (type) {
     case kF32: return launch_float_t<kF32>(w, x, y, ldy, rows, width, row_bytes, m, stream);
     case kF16: return launch_float_t<kF16>(w, x, y, ldy, rows, width, row_bytes, m, stream);
@@ -452,6 +449,33 @@ bool launch_gemm_float(int type, uint32_t m, const uint8_t *w, const float *x, f
     case kQ6K: return launch_float_t<kQ6K>(w, x, y, ldy, rows, width, row_bytes, m, stream);
     default: return false;
     }
+}
+
+}  // namespace
+
+bool launch_gemm_float(int type, uint32_t m, const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows,
+                       uint32_t width, hipStream_t stream)
+{
+    uint32_t e = 0, b = 0;
+    if (m < 1 || ldy < rows || !rows || !width || !format_block_shape(type, &e, &b) || width % e) return false;
+    const uint64_t row_bytes = (uint64_t)width / e * b;
+    /* a workgroup addresses its rows with 32-bit offsets and a launch's grid
+     * holds 65535 token tiles: wider rows and longer batches take several
+     * launches (with one row per launch the stride is not used) */
+    const uint64_t fit = 0xffffffffull / row_bytes;
+    const uint32_t row_step = fit >= kFloatRows ? rows : fit ? (uint32_t)fit : 1u, token_step = 65535u * 64;
+    for (uint32_t r = 0; r < rows;) {
+        const uint32_t nr = rows - r < row_step ? rows - r : row_step;
+        for (uint32_t t = 0; t < m;) {
+            const uint32_t nt = m - t < token_step ? m - t : token_step;
+            if (!launch_float_rows(type, nt, w + (size_t)r * row_bytes, x + (size_t)t * width,
+                                   y + (size_t)t * ldy + r, ldy, nr, width, (uint32_t)row_bytes, stream))
+                return false;
+            t += nt;
+        }
+        r += nr;
+    }
+    return true;
 }
 
 }  // namespace q38
