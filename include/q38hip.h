@@ -139,9 +139,9 @@ int q38hip_quantize_q8_k(Q38Q8KBlock *output, const float *input,
 
 /* Device form of q38_tensor_gemm_q8_k (src/qwen38/qwen38_quant.c:2950-3169);
  * batch_size = 1 is q38_tensor_gemv_q8_k (:2833-2922).  Any batch_size >= 1:
- * the kernels take up to 8 tokens per launch, and larger batches run as
- * consecutive launches over token chunks (every token's outputs are
- * independent of the rest of the batch, so the bits are those of one call). */
+ * up to 8 tokens and prompt batches take one launch; shapes without a prompt
+ * kernel run as consecutive launches of up to 8 tokens (every token's outputs
+ * are independent of the rest of the batch, so the bits are the same). */
 int q38hip_gemm_q8_k(float *output, const Q38Q8KBlock *input,
                      uint32_t batch_size, uint64_t input_length,
                      const Q38GGUFTensor *tensor, void *stream);

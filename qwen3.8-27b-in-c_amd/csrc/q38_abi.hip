@@ -213,10 +213,10 @@ int q38hip_gemm_q8_k(float *output, const Q38Q8KBlock *input, uint32_t batch_siz
     if (!check_gemm(output, input, batch_size, input_length, tensor)) return 0;
     DeviceState *state = device_state();
     if (!state) return fail("device initialisation failed");
-    /* Any batch size, as the reference (qwen38_quant.c:2950-2956): the
-     * kernels take up to 8 tokens per launch and every token's row results
-     * are independent of the others in the batch, so consecutive launches
-     * over token chunks give the same bits as one. */
+    /* Any batch size, as the reference (qwen38_quant.c:2950-2956): a prompt
+     * kernel takes the whole batch where there is one, else launches of up to
+     * 8 tokens; every token's row results are independent of the others in
+     * the batch, so the bits are the same. */
     const uint32_t rows = (uint32_t)tensor->shape[1], nb = (uint32_t)(input_length / 256);
     /* IQ1_M prefill batches: one launch of the 256 x 64 matrix-core tiles */
     if (tensor->type == q38::kIQ1M && batch_size >= (uint32_t)q38::kWideMinTokens &&
