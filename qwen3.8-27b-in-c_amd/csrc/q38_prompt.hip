@@ -23,8 +23,11 @@
  * activations of group g: one more product per lane, added with one fmaf
  * (both terms are exact, so it rounds as the integer's conversion does).
  * Min and correction sums (m[i] * S[i]) are products over the 16 sums (Q4_K:
- * their int16 pair sums), each split into a multiple of 64 and a rest, which
- * are exact for any int16.
+ * their int16 pair sums), each split into a multiple of 64 and a rest, both
+ * exact in fp16.  Their sums stay below 2^24 for any int16 (16 * 15 * 32768 for
+ * Q2_K and IQ1_S, 2 * 63 * 32768 for a Q4_K lane's two sub-blocks) but for
+ * Q5_K's 16 * 63 * 32768: there the multiples of 64 and the rests are summed
+ * apart, below 2^19 steps of 64 and 2^16.
  * IQ4_NL has one fp32 scale per group, so each group's product is taken by
  * itself (v_mfma_f32_32x32x4_2b_f16: two groups per instruction).
  *
@@ -458,12 +461,27 @@ __global__ __launch_bounds__(kPromptThreads, 1) void gemm_prompt(const uint8_t *
                 }
                 if constexpr (P::scalar) {
                     if (lh == (kSub == 2 ? u : 1)) {
+                        auto sums4 = [&](int k) {
+                            return *reinterpret_cast<const half4p *>(lds + L::ss + (k * kTok + 32 * tt + r) * 8);
+                        };
+                        auto factors4 = [&](int k) {
+                            return *reinterpret_cast<const half4p *>(lds + L::ms + (k * kPromptRows + wrow) * 8);
+                        };
                         f16v m = {};
+                        if constexpr (T == kQ5K) {
+                            f16v low = {};
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const half4p sa = *reinterpret_cast<const half4p *>(lds + L::ss + ((4 * q + i) * kTok + 32 * tt + r) * 8);
-                            const half4p sb = *reinterpret_cast<const half4p *>(lds + L::ms + (i * kPromptRows + wrow) * 8);
-                            m = __builtin_amdgcn_mfma_f32_32x32x8f16(sa, sb, m, 0, 0, 0);
+                            for (int i = 0; i < 2; ++i) {
+                                m = __builtin_amdgcn_mfma_f32_32x32x8f16(sums4(2 * i + q), factors4(2 * i + q), m, 0, 0, 0);
+                                low = __builtin_amdgcn_mfma_f32_32x32x8f16(sums4(4 + 2 * i + q), factors4(2 * i + q), low, 0, 0, 0);
+                            }
+                            /* both exact: one rounding, as the integer sum's conversion */
+#pragma unroll
+                            for (int j = 0; j < 16; ++j) m[j] = fadd_rn(m[j], low[j]);
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                m = __builtin_amdgcn_mfma_f32_32x32x8f16(sums4(4 * q + i), factors4(i), m, 0, 0, 0);
                         }
 #pragma unroll
                         for (int j = 0; j < 16; ++j) {

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import format_cases as fc
-from oracle import FORMAT_NAMES, IQ1_M, Q8K_DTYPE, Q8K_FORMATS
+from oracle import FORMAT_NAMES, IQ1_M, IQ1_S, Q2_K, Q4_K, Q5_K, Q8K_DTYPE, Q8K_FORMATS
 
 pytestmark = [pytest.mark.gpu, pytest.mark.timeout(600)]
 
@@ -58,4 +58,26 @@ def test_prompt_extreme_fields_match_oracle(device, oracle, qtype):
     q8["quants"][:8] = 127              # whole blocks of one sign: the largest sums
     q8["quants"][8:16] = -128
     q8["sums"] = rng.choice([-32768, -2048, -1, 63, 2047, 32767], q8["sums"].shape)
+    check(device, oracle, qtype, rows, width, data.reshape(-1), q8, tokens)
+
+
+@pytest.mark.parametrize("qtype", (Q2_K, Q4_K, Q5_K, IQ1_S), ids=lambda t: FORMAT_NAMES[t])
+def test_prompt_sums_of_one_sign_match_oracle(device, oracle, qtype):
+    """Blocks whose sixteen sums lie at one end of int16: the min or correction
+    sum of a block is then at its largest (Q5_K: 16 x 63 x 32768, twice 2^24),
+    and is rounded once, when it becomes a float.  Some rows have the largest
+    multipliers; the sums differ in their low bits, so that a sum that is
+    rounded on the way shows."""
+    rng = np.random.default_rng(850 + qtype)
+    rows, width, tokens = 70, 768, 37
+    data = fc.random_matrix(qtype, rows, width, rng).reshape(rows, -1)
+    if qtype in (Q4_K, Q5_K):
+        block = fc.FORMATS[qtype][1]
+        for start in range(0, data.shape[1], block):
+            data[:35, start + 4:start + 16] |= rng.integers(240, 256, (35, 12), dtype=np.uint8)
+    q8 = np.zeros(tokens * width // 256, dtype=Q8K_DTYPE)
+    q8["scale"] = rng.uniform(-0.1, 0.1, q8.size)
+    q8["quants"] = rng.integers(-127, 128, q8["quants"].shape)
+    q8["sums"] = 32767 - rng.integers(0, 200, q8["sums"].shape)
+    q8["sums"][::2] = rng.integers(0, 200, q8["sums"][::2].shape) - 32768
     check(device, oracle, qtype, rows, width, data.reshape(-1), q8, tokens)
