@@ -223,10 +223,12 @@ int q38hip_gemm_q8_k(float *output, const Q38Q8KBlock *input, uint32_t batch_siz
         q38::launch_gemm_iq1m_wide(batch_size, tensor->data, reinterpret_cast<const uint8_t *>(input), output, rows,
                                    rows, nb, state->grid, static_cast<hipStream_t>(stream)))
         return 1;
-    if (batch_size >= (uint32_t)q38::kWideMinTokens &&
-        q38::launch_gemm_prompt((int)tensor->type, batch_size, tensor->data, reinterpret_cast<const uint8_t *>(input),
-                                output, rows, rows, nb, state->grid, static_cast<hipStream_t>(stream)))
-        return 1;
+    if (q38::prompt_takes((int)tensor->type, batch_size, rows, nb))
+        return q38::launch_gemm_prompt((int)tensor->type, batch_size, tensor->data,
+                                       reinterpret_cast<const uint8_t *>(input), output, rows, rows, nb, state->grid,
+                                       static_cast<hipStream_t>(stream))
+                   ? 1
+                   : fail("prompt GEMM launch failed");
     for (uint32_t t0 = 0; t0 < batch_size;) {
         const uint32_t n = token_chunk(batch_size - t0, 1);
         const uint8_t *x = reinterpret_cast<const uint8_t *>(input) + (size_t)t0 * nb * sizeof(Q38Q8KBlock);
@@ -262,7 +264,7 @@ int q38hip_gemm_f32(float *output, const float *input, uint32_t batch_size, uint
     }
     if (!q38::launch_gemm_float((int)tensor->type, batch_size, tensor->data, input, output, rows, rows,
                                 (uint32_t)input_length, s))
-        return fail("unsupported float GEMM configuration");
+        return fail("float GEMM launch failed");
     return 1;
 }
 

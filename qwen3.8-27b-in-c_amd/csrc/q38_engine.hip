@@ -847,9 +847,9 @@ bool gemm_rows(Q38Model *m, const DevTensor &w, uint32_t count, const uint8_t *x
     if (w.type == IQ1_M && count >= (uint32_t)q38::kWideMinTokens &&
         q38::launch_gemm_iq1m_wide(count, wdata, x, out, ldy, rows, nb, m->grid, m->stream))
         return true;
-    if (count >= (uint32_t)q38::kWideMinTokens &&
-        q38::launch_gemm_prompt((int)w.type, count, wdata, x, out, ldy, rows, nb, m->grid, m->stream))
-        return true;
+    if (q38::prompt_takes((int)w.type, count, rows, nb))
+        return q38::launch_gemm_prompt((int)w.type, count, wdata, x, out, ldy, rows, nb, m->grid, m->stream) ||
+               report("prompt GEMM launch failed");
     /* Q4_K, Q6_K and IQ1_M have their own kernel families; the other Q8_K
      * formats run the generic lane-chain kernel */
     const bool tuned = w.type == Q4_K || w.type == Q6_K || w.type == IQ1_M;

@@ -389,10 +389,9 @@ template <int T, int MT, int CW, int ST = 64>
 bool launch_float(const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows, uint32_t width,
                   uint32_t row_bytes, uint32_t tokens, hipStream_t stream)
 {
-    hipLaunchKernelGGL((gemm_float_kernel<T, MT, CW, ST>),
-                       dim3((rows + kFloatRows - 1) / kFloatRows, (tokens + MT * CW - 1) / (MT * CW)),
-                       dim3(64 * CW + kProducers), 0, stream, w, x, y, ldy, rows, width, row_bytes, tokens);
-    return hipGetLastError() == hipSuccess;
+    return launch_kernel(gemm_float_kernel<T, MT, CW, ST>,
+                         dim3((rows + kFloatRows - 1) / kFloatRows, (tokens + MT * CW - 1) / (MT * CW)),
+                         dim3(64 * CW + kProducers), stream, w, x, y, ldy, rows, width, row_bytes, tokens);
 }
 
 /* Up to eight tokens.  The types of real float matrices (GGUF files keep

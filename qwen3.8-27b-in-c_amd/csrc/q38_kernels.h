@@ -4,7 +4,24 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <tuple>
+
 namespace q38 {
+
+/* one kernel launch, and whether it was accepted.  The status is the launch's
+ * own: an error that the thread's earlier HIP calls left behind is neither
+ * taken for it nor cleared. */
+template <typename... Params, typename... Args>
+bool launch_kernel(void (*kernel)(Params...), dim3 grid, dim3 block, hipStream_t stream, Args... args)
+{
+    std::tuple<Params...> values(args...);
+    return std::apply(
+        [&](auto &...v) {
+            void *pointers[] = {&v...};
+            return hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, pointers, 0, stream) == hipSuccess;
+        },
+        values);
+}
 
 /* state slots of each recurrent layer: one more than the largest batch */
 constexpr uint32_t kRecurrentStateSlots = 9;
@@ -81,9 +98,11 @@ bool format_takes_q8k(int type);
 bool format_row_decodable(int type);
 bool launch_gemm_format(int type, int m, const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy, uint32_t rows,
                         uint32_t nb, const void *grid, hipStream_t stream);
-/* q38_prompt.hip: the same products for a prompt batch of any length (from
- * kWideMinTokens tokens on), and for row-major Q4_K and Q6_K; false for other
- * types and for sizes past its 32-bit offsets */
+/* q38_prompt.hip: the same products for a prompt batch, and for row-major Q4_K
+ * and Q6_K.  prompt_takes: whether it is the kernel for such a batch (from
+ * kWideMinTokens tokens on; not for other types and for sizes past its 32-bit
+ * offsets); launch_gemm_prompt: false when the launch failed. */
+bool prompt_takes(int type, uint32_t tokens, uint32_t rows, uint32_t nb);
 bool launch_gemm_prompt(int type, uint32_t tokens, const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy,
                         uint32_t rows, uint32_t nb, const void *grid, hipStream_t stream);
 bool launch_gemm_float(int type, uint32_t m, const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows,

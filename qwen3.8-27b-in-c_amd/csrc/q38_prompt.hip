@@ -544,11 +544,10 @@ bool launch_prompt(const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy, u
                    uint32_t tokens, const void *grid, hipStream_t stream)
 {
     static_assert(PromptLds<T, TT>::bytes <= 160 * 1024, "LDS");
-    hipLaunchKernelGGL((gemm_prompt<T, TT>),
-                       dim3((rows + kPromptRows - 1) / kPromptRows, (tokens + 32 * TT - 1) / (32 * TT)),
-                       dim3(kPromptThreads), 0, stream, w, x, y, ldy, rows, nb, tokens,
-                       static_cast<const uint32_t *>(grid));
-    return hipGetLastError() == hipSuccess;
+    return launch_kernel(gemm_prompt<T, TT>,
+                         dim3((rows + kPromptRows - 1) / kPromptRows, (tokens + 32 * TT - 1) / (32 * TT)),
+                         dim3(kPromptThreads), stream, w, x, y, ldy, rows, nb, tokens,
+                         static_cast<const uint32_t *>(grid));
 }
 
 /* Workgroups of 128 tokens where their registers hold (no min lanes, offset
@@ -574,18 +573,24 @@ bool launch_prompt_t(const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy,
 
 }  // namespace
 
-bool launch_gemm_prompt(int type, uint32_t tokens, const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy,
-                        uint32_t rows, uint32_t nb, const void *grid, hipStream_t stream)
+bool prompt_takes(int type, uint32_t tokens, uint32_t rows, uint32_t nb)
 {
+    if (!format_takes_q8k(type) || type == kIQ1M || !rows || !nb || tokens < (uint32_t)kWideMinTokens) return false;
     /* 32-bit byte offsets inside a workgroup's rows, and the grid's limits */
-    if (!rows || !nb || !tokens || ldy < rows || nb > 65536 || tokens > 65535u * 64) return false;
+    if (nb > 65536 || tokens > 65535u * 64) return false;
     /* Q4_K and Q6_K have kernels for up to 8 tokens that beat a round of these
      * workgroups (2.1 / 3.1 us per block column whatever the token count) on
      * matrices too small to fill the chip: 1024 x 5120, 9 / 17 / 33 tokens 22 /
      * 38 / 70 us in launches of 8 against 43 us (Q4_K), 25 / 43 / 79 against 61
      * us (Q6_K).  From 4096 rows on they lose at 9 tokens already (34816 x
      * 5120: 370 against 128 us and 337 against 184 us). */
-    if ((type == kQ4K || type == kQ6K) && rows < 4096 && tokens < 24) return false;
+    return !((type == kQ4K || type == kQ6K) && rows < 4096 && tokens < 24);
+}
+
+bool launch_gemm_prompt(int type, uint32_t tokens, const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy,
+                        uint32_t rows, uint32_t nb, const void *grid, hipStream_t stream)
+{
+    if (ldy < rows || !prompt_takes(type, tokens, rows, nb)) return false;
     switch (type) {
     case kQ2K: return launch_prompt_t<kQ2K>(w, x, y, ldy, rows, nb, tokens, grid, stream);
     case kQ3K: return launch_prompt_t<kQ3K>(w, x, y, ldy, rows, nb, tokens, grid, stream);
