@@ -400,11 +400,6 @@ struct Q38Model {
      * and the sampler's candidate lists */
     const float *last_logits = nullptr;
     uint8_t *presence = nullptr, *sample_scratch = nullptr;
-    /* a prompt batch's converted activations (Q4_K tiled matrices), and the
-     * buffer's size */
-    uint8_t *wide_operands = nullptr;
-    size_t wide_operand_size = 0;
-    bool tiled_q4k = false;
     /* host side */
     float *host_logits = nullptr;
     uint32_t *host_words = nullptr;
@@ -675,7 +670,6 @@ void release(Q38Model *m)
     dfree(m->q8k);
     dfree(m->presence);
     dfree(m->sample_scratch);
-    dfree(m->wide_operands);
     if (m->weights) (void)hipFree(m->weights);
     if (m->mtp_weights) (void)hipFree(m->mtp_weights);
     if (m->tiled_weights) (void)hipFree(m->tiled_weights);
@@ -699,13 +693,6 @@ bool allocate_state(Q38Model *m)
     m->prefill_rows = (uint32_t)std::max<size_t>(kBatch, std::min<size_t>(kPrefillRows, by_scores));
     m->scratch_rows = std::max(kBatch, m->prefill_rows);
     const uint32_t B = m->scratch_rows;
-    /* the longest prompt batch over the widest matrix (142 MB at 4096 rows);
-     * every step runs on the model's one stream */
-    if (m->tiled_q4k) {
-        const size_t bytes = q38::wide_operand_bytes(B, kFFN / 256);
-        if (!dalloc(&m->wide_operands, bytes)) return false;
-        m->wide_operand_size = bytes;
-    }
     const size_t slots = q38::kRecurrentStateSlots;
     bool ok = dalloc(&m->conv_state, slots * conv_count()) && dalloc(&m->delta_state, slots * delta_count()) &&
               dalloc(&m->key_cache, kv_count(ctx)) && dalloc(&m->value_cache, kFullLayers * value_layer_floats(ctx)) &&
@@ -884,10 +871,15 @@ bool gemm_tiled(Q38Model *m, const DevTensor &w, uint32_t count, const uint8_t *
 {
     if (!w.tiled) return false;
     const uint32_t nb = (uint32_t)(w.width / 256);
-    if (w.type == Q4_K && count >= (uint32_t)q38::kWideMinTokens)
+    if (w.type == Q4_K && count >= (uint32_t)q38::kWideMinTokens) {
+        /* the converted activations lie in the attention's score rows: these
+         * are written and read inside launch_attention only, on this stream,
+         * and hold them for every batch of 9 to scratch_rows tokens (34816
+         * bytes a token at most, against 96 a token and context position) */
+        const size_t room = (size_t)m->scratch_rows * kAttnHeads * m->context_length * sizeof(float);
         return q38::launch_gemm_q4k_wide(count, w.tiled, x, out, ldy, rows, nb, m->stream,
-                                         q38::wide_operand_bytes(count, nb) <= m->wide_operand_size ? m->wide_operands
-                                                                                                    : nullptr);
+                                         q38::wide_operand_bytes(count, nb) <= room ? m->scores : nullptr);
+    }
     if (w.type == Q4_K)
         return count >= 1 && q38::launch_gemm_q4k_tiled((int)count, w.tiled, x, out, ldy, rows, nb, m->stream);
     if (w.type == IQ1_M)
@@ -988,7 +980,6 @@ bool build_tiled(Q38Model *m, uint32_t first, uint32_t last, bool with_eh, void 
     }
     if (!total) return true;
     if (!hip_ok(hipMalloc(mem, total), "tiled weight allocation")) return false;
-    for (const Job &j : jobs) m->tiled_q4k |= j.type == Q4_K;
     uint8_t *base = static_cast<uint8_t *>(*mem);
     for (size_t k = 0; k < jobs.size(); ++k) {
         const Job &j = jobs[k];

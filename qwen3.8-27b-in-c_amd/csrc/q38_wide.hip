@@ -43,9 +43,9 @@
  * 34816 x 5120 611 / 519 / 489 us (373 TFLOP/s), 5120 x 17408 334 / 274 / 257,
  * 16480 x 5120 325 / 273 / 258, 5120 x 6144 127 / 105 / 99 us; converting with
  * fp16 min products 585 us (34816 x 5120) and 311 us (5120 x 17408).  The
- * engine keeps the operand buffer; callers without a workspace (the C ABI's
- * one-call GEMM) take the converting form, since the buffer would have to be
- * allocated on each call.
+ * engine lends its attention score rows for the operands; callers without a
+ * workspace (the C ABI's one-call GEMM) take the converting form, since the
+ * buffer would have to be allocated on each call.
  */
 #include "q38_device.h"
 #include "q38_kernels.h"
