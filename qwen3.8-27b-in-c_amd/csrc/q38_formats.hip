@@ -69,6 +69,7 @@ __global__ __launch_bounds__(64 * H) void gemv_format_kernel(const uint8_t *__re
                                                                 uint32_t phase_blocks,
                                                                 const uint32_t *__restrict__ iq1s_grid)
 {
+    static_assert(T != kIQ4NL, "IQ4_NL has a scale per group: gemv_nl_kernel");
     using F = GemvFormat<T, MT>;
     constexpr uint32_t kBytes = block_bytes<T>();
     constexpr int kMine = (MT + H - 1) / H;   /* tokens whose chains a wavefront runs */
@@ -207,12 +208,13 @@ void launch_format_typed(const uint8_t *w, const uint8_t *x, float *y, uint32_t 
 {
     if constexpr (T == kIQ4NL) {
         hipLaunchKernelGGL(gemv_nl_kernel<MT>, dim3((rows + 31) / 32), dim3(256), 0, stream, w, x, y, ldy, rows, nb);
-        return;
+    } else {
+        using F = GemvFormat<T, MT>;
+        const uint32_t phases = (nb + F::kBlocks - 1) / F::kBlocks, blocks = (nb + phases - 1) / phases;
+        hipLaunchKernelGGL((gemv_format_kernel<T, MT, H>), dim3((rows + 7) / 8), dim3(64 * H),
+                           F::table + blocks * F::per_block, stream, w, x, y, ldy, rows, nb, blocks,
+                           static_cast<const uint32_t *>(grid));
     }
-    using F = GemvFormat<T, MT>;
-    const uint32_t phases = (nb + F::kBlocks - 1) / F::kBlocks, blocks = (nb + phases - 1) / phases;
-    hipLaunchKernelGGL((gemv_format_kernel<T, MT, H>), dim3((rows + 7) / 8), dim3(64 * H), F::table + blocks * F::per_block,
-                       stream, w, x, y, ldy, rows, nb, blocks, static_cast<const uint32_t *>(grid));
 }
 
 template <int T>
