@@ -62,6 +62,15 @@ struct GemvFormat {
     static constexpr int kBlocks = (64 * 1024 - table) / per_block;           /* blocks of a phase at most */
 };
 
+/* the block's integer min or correction sum of the lane's row: two products
+ * per lane, added over the row's eight lanes */
+__device__ __forceinline__ int row_extra(const uint8_t *xb, int l, int m0, int m1)
+{
+    const int pair = *reinterpret_cast<const int *>(xb + 260 + 4 * l);
+    const int sum = quad_sum(m0 * (int)(int16_t)pair + m1 * (pair >> 16));
+    return sum + dpp_move<0x141>(0, sum);   /* the row's other quad */
+}
+
 template <int T, int MT, int H>
 __global__ __launch_bounds__(64 * H) void gemv_format_kernel(const uint8_t *__restrict__ w,
                                                                 const uint8_t *__restrict__ x, float *__restrict__ y,
@@ -69,7 +78,7 @@ __global__ __launch_bounds__(64 * H) void gemv_format_kernel(const uint8_t *__re
                                                                 uint32_t phase_blocks,
                                                                 const uint32_t *__restrict__ iq1s_grid)
 {
-    static_assert(T != kIQ4NL, "IQ4_NL has a scale per group: gemv_nl_kernel");
+    static_assert(T != kIQ4NL, "IQ4_NL has a scale per group: gemv_rows_kernel");
     using F = GemvFormat<T, MT>;
     constexpr uint32_t kBytes = block_bytes<T>();
     constexpr int kMine = (MT + H - 1) / H;   /* tokens whose chains a wavefront runs */
@@ -114,11 +123,7 @@ __global__ __launch_bounds__(64 * H) void gemv_format_kernel(const uint8_t *__re
                 for (int g = 0; g < 8; ++g) wsum = mad24(lb.s[g], dot4z((int)lb.q[g], aq[8 * g]), wsum);
                 *so = (float)wsum;
                 int extra = 0;
-                if constexpr (has_extra<T>()) {
-                    const int pair = *reinterpret_cast<const int *>(xb + 260 + 4 * l);
-                    extra = quad_sum(m0 * (int)(int16_t)pair + m1 * (pair >> 16));
-                    extra += dpp_move<0x141>(0, extra);   /* the row's other quad */
-                }
+                if constexpr (has_extra<T>()) extra = row_extra(xb, l, m0, m1);
                 if (l == 0) {
                     const float d = fmul_rn(lb.d, xs);
                     co[0] = d;
@@ -161,36 +166,137 @@ __global__ __launch_bounds__(64 * H) void gemv_format_kernel(const uint8_t *__re
     }
 }
 
-/* IQ4_NL takes one fma per 32-element group instead of one per block, so
- * handing sums through LDS would cost eight times as much (34816 x 5120, one
- * token: 83 against 44 us): eight lanes per row, each running its chain over
- * all blocks. */
-template <int MT>
-__global__ __launch_bounds__(256) void gemv_nl_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ x,
-                                                      float *__restrict__ y, uint32_t ldy, uint32_t rows, uint32_t nb)
+/* decode_lane for gemv_rows_kernel: with few blocks to a row, formats with
+ * several header fields per group are faster loading the bytes a lane uses than
+ * whole headers to shift them from (65536 x 1024, one token: IQ2_S 27 against
+ * 32 us, IQ1_S 26 against 28 us) */
+template <int T>
+__device__ __forceinline__ void decode_walk(const uint8_t *blk, int l, const uint32_t *table, LaneBlock &b)
+{
+    const int sec = l >> 1, half = l & 1;
+    if constexpr (T == kIQ2S) {
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            const uint32_t index = blk[2 + 4 * g + sec] | (((uint32_t)blk[66 + g] << (8 - 2 * sec)) & 0x300u);
+            b.q[g] = negate_bytes(table[2 * index + half], byte_mask4((uint32_t)blk[34 + 4 * g + sec] >> (4 * half)));
+            b.s[g] = 1 + 2 * (int)(((uint32_t)blk[74 + g] >> (l & 4)) & 15u);
+        }
+        b.d = 0.125f * f16_to_f32(ld16(blk));
+    } else if constexpr (T == kIQ3S) {
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            const uint32_t index = blk[2 + 8 * g + l] | (((uint32_t)(blk[66 + g] >> l) & 1u) << 8);
+            b.q[g] = negate_bytes(table[index], byte_mask4((uint32_t)blk[74 + 4 * g + sec] >> (4 * half)));
+            b.s[g] = 1 + 2 * (int)((blk[106 + g / 2] >> (4 * (g & 1))) & 15u);
+        }
+        b.d = f16_to_f32(ld16(blk));
+    } else if constexpr (T == kIQ1S) {
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            const uint32_t high = ld16(blk + 34 + 2 * g);
+            const uint32_t index = blk[2 + 4 * g + sec] | (((high >> (3 * sec)) & 7u) << 8);
+            b.q[g] = table[2 * index + half];
+            b.s[g] = 1 + 2 * (int)((high >> 12) & 7u);
+        }
+        b.d = f16_to_f32(ld16(blk));
+    } else if constexpr (T == kQ3K) {
+        const int hi = l >= 4;
+        const uint32_t hm = ld32u(blk + 4 * l);
+        const uint32_t d0 = ld32u(blk + 32 + 4 * l), d1 = ld32u(blk + 64 + 4 * l);
+        const uint8_t *sc = blk + 96;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            const uint32_t low = ((g < 4 ? d0 : d1) >> (2 * (g & 3))) & 0x03030303u;
+            const uint32_t absent = ~(hm >> g) & 0x01010101u;
+            b.q[g] = low + absent * 0xfcu;
+            const int i = 2 * g + hi;
+            const int lo4 = g < 4 ? sc[i] & 15 : sc[i - 8] >> 4;
+            const int hi2 = (sc[8 + i % 4] >> (2 * (i / 4))) & 3;
+            b.s[g] = (lo4 | hi2 << 4) - 32;
+        }
+        b.d = f16_to_f32(ld16(blk + 108));
+    } else {
+        decode_lane<T>(blk, l, table, b);
+    }
+}
+
+/* The same for short rows of tall matrices, and for IQ4_NL at any length:
+ * eight lanes per row, each running its chain over all blocks, 32 rows per
+ * workgroup, the codebooks read from global memory.  Where rows fill the chip
+ * by themselves, a workgroup per eight of them costs more than it spreads: its
+ * wavefronts have a block each or none, and every one copies the codebook
+ * (IQ1_S 16 KB, IQ2_S 8 KB).  IQ4_NL takes one fma per 32-element group instead
+ * of one per block, so handing its sums through LDS would cost eight times as
+ * much (34816 x 5120, one token: 83 against 44 us).
+ *
+ * walk_rows says which: the row walk pays from about 2700 rows per block of a
+ * row on (block ranges / row walk: 65536 x 256, one and five tokens, Q3_K 12.2 /
+ * 4.4 and 32.9 / 8.0 us, IQ1_S 17.2 / 7.7 and 45.4 / 11.3; 8192 x 768, five
+ * tokens, Q3_K 6.4 / 5.7), up to as many blocks as where the codebook in LDS
+ * or, from four tokens on, the shared activations win again (65536 x 1536 and
+ * 65536 x 5120, one token, IQ2_S 41 / 39 and 96 / 127 us; 65536 x 5120 Q3_K 54 /
+ * 48; 65536 x 2048 and 65536 x 3072, five tokens, IQ2_S 78 / 73 and 98 / 108).
+ * An IQ1_S walk is still 3 to 9 % behind the kernel that stood here before the
+ * block ranges (65536 x 256, five tokens 10.5 us). */
+template <int T, int MT>
+bool walk_rows(uint32_t rows, uint32_t nb)
+{
+    constexpr bool book = table_dwords<T>() > 0;
+    const uint32_t most = book ? (MT > 3 ? 6 : 4) + (rows >= 65536 ? 2 : 0) : MT > 3 ? 10 : 20;
+    return T == kIQ4NL || (nb <= most && rows >= 2700 * nb);
+}
+
+/* eight tokens: in the registers of eight wavefronts per SIMD the compiler
+ * orders the loads one after another (Q5_K 65536 x 768 57 against 29 us) */
+template <int T, int MT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, MT == 8 ? 6 : 8)))
+void gemv_rows_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ x, float *__restrict__ y, uint32_t ldy,
+                      uint32_t rows, uint32_t nb, const uint32_t *__restrict__ iq1s_grid)
 {
     const int l = threadIdx.x & 7;
-    const uint32_t row = (blockIdx.x * 256u + threadIdx.x) >> 3;
-    const uint8_t *wr = w + (size_t)(row < rows ? row : rows - 1) * nb * block_bytes<kIQ4NL>();
-    float acc[MT];
+    const uint32_t row = blockIdx.x * 32u + (threadIdx.x >> 3);
+    const uint8_t *wr = w + (size_t)(row < rows ? row : rows - 1) * nb * block_bytes<T>();
+    const uint32_t *table = table_of<T>(iq1s_grid);
+    float acc[MT], scalar[MT];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) acc[t] = 0.0f;
+    for (int t = 0; t < MT; ++t) acc[t] = scalar[t] = 0.0f;
     for (uint32_t b = 0; b < nb; ++b) {
+        const uint8_t *blk = wr + (size_t)b * block_bytes<T>();
         LaneBlock lb;
-        decode_lane<kIQ4NL>(wr + (size_t)b * block_bytes<kIQ4NL>(), l, nullptr, lb);
+        decode_walk<T>(blk, l, table, lb);
+        int m0 = 0, m1 = 0;
+        if constexpr (has_extra<T>()) extra_factors<T>(blk, l, m0, m1);
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             const uint8_t *xb = x + ((size_t)t * nb + b) * kQ8KBytes;
             const float xs = *reinterpret_cast<const float *>(xb);
             const int *aq = reinterpret_cast<const int *>(xb + 4) + l;
+            if constexpr (T == kIQ4NL) {
 #pragma unroll
-            for (int g = 0; g < 8; ++g)
-                acc[t] = __builtin_fmaf(fmul_rn(lb.gd[g], xs), (float)dot4z((int)lb.q[g], aq[8 * g]), acc[t]);
-            /* from five tokens on the compiler would move the links past the
-             * other tokens and keep their products in registers (eight tokens,
-             * 34816 x 5120: 353 against 117 us); below, its order is the
-             * faster one (three tokens, 17408 columns: 70 against 113 us) */
-            if constexpr (MT > 4) asm volatile("" : "+v"(acc[t]));
+                for (int g = 0; g < 8; ++g)
+                    acc[t] = __builtin_fmaf(fmul_rn(lb.gd[g], xs), (float)dot4z((int)lb.q[g], aq[8 * g]), acc[t]);
+                /* from five tokens on the compiler would move the links past
+                 * the other tokens and keep their products in registers (eight
+                 * tokens, 34816 x 5120: 353 against 117 us); below, its order
+                 * is the faster one (three tokens, 17408 columns: 70 against
+                 * 113 us) */
+                if constexpr (MT > 4) asm volatile("" : "+v"(acc[t]));
+            } else {
+                int wsum = 0;
+#pragma unroll
+                for (int g = 0; g < 8; ++g) wsum = mad24(lb.s[g], dot4z((int)lb.q[g], aq[8 * g]), wsum);
+                const float d = fmul_rn(lb.d, xs);
+                acc[t] = __builtin_fmaf(d, (float)wsum, acc[t]);
+                if constexpr (has_extra<T>()) {
+                    const float extra = (float)row_extra(xb, l, m0, m1);
+                    if constexpr (T == kIQ1S) scalar[t] = fadd_rn(scalar[t], fmul_rn(d, extra));
+                    else scalar[t] = __builtin_fmaf(-fmul_rn(lb.dmin, xs), extra, scalar[t]);
+                }
+                if constexpr (MT > 3) {
+                    if constexpr (has_extra<T>()) asm volatile("" : "+v"(acc[t]), "+v"(scalar[t]));
+                    else asm volatile("" : "+v"(acc[t]));
+                }
+            }
         }
     }
 #pragma unroll
@@ -198,6 +304,8 @@ __global__ __launch_bounds__(256) void gemv_nl_kernel(const uint8_t *__restrict_
         float v = fadd_rn(acc[t], __shfl_xor(acc[t], 4, 64));
         v = fadd_rn(v, __shfl_xor(v, 2, 64));
         v = fadd_rn(v, __shfl_xor(v, 1, 64));
+        if constexpr (T == kIQ1S) v = fadd_rn(v, fmul_rn(0.125f, scalar[t]));
+        else if constexpr (has_extra<T>()) v = fadd_rn(v, scalar[t]);
         if (l == 0 && row < rows) y[(size_t)t * ldy + row] = v;
     }
 }
@@ -206,15 +314,18 @@ template <int T, int MT, int H>
 void launch_format_typed(const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy, uint32_t rows, uint32_t nb,
                          const void *grid, hipStream_t stream)
 {
-    if constexpr (T == kIQ4NL) {
-        hipLaunchKernelGGL(gemv_nl_kernel<MT>, dim3((rows + 31) / 32), dim3(256), 0, stream, w, x, y, ldy, rows, nb);
-    } else {
-        using F = GemvFormat<T, MT>;
-        const uint32_t phases = (nb + F::kBlocks - 1) / F::kBlocks, blocks = (nb + phases - 1) / phases;
-        hipLaunchKernelGGL((gemv_format_kernel<T, MT, H>), dim3((rows + 7) / 8), dim3(64 * H),
-                           F::table + blocks * F::per_block, stream, w, x, y, ldy, rows, nb, blocks,
-                           static_cast<const uint32_t *>(grid));
+    const uint32_t *iq1s = static_cast<const uint32_t *>(grid);
+    if constexpr (T != kIQ4NL) {
+        if (!walk_rows<T, MT>(rows, nb)) {
+            using F = GemvFormat<T, MT>;
+            const uint32_t phases = (nb + F::kBlocks - 1) / F::kBlocks, blocks = (nb + phases - 1) / phases;
+            hipLaunchKernelGGL((gemv_format_kernel<T, MT, H>), dim3((rows + 7) / 8), dim3(64 * H),
+                               F::table + blocks * F::per_block, stream, w, x, y, ldy, rows, nb, blocks, iq1s);
+            return;
+        }
     }
+    hipLaunchKernelGGL((gemv_rows_kernel<T, MT>), dim3((rows + 31) / 32), dim3(256), 0, stream, w, x, y, ldy, rows, nb,
+                       iq1s);
 }
 
 template <int T>

@@ -1,0 +1,58 @@
+"""Times of calls that once lost to the kernels they replaced.  Each bound
+lies between the two: the call takes at most two thirds of it, the form that
+was mended takes over a quarter more.  Best of several runs, GPU events."""
+import ctypes
+
+import pytest
+
+pytestmark = [pytest.mark.gpu, pytest.mark.timeout(300)]
+
+
+def best_us(call, calls=40, runs=7):
+    import torch
+    call()
+    best = 1e30
+    for _ in range(runs):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        torch.cuda.synchronize()
+        start.record()
+        for _ in range(calls):
+            call()
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, start.elapsed_time(end) / calls * 1e3)
+    return best
+
+
+def product(device, qtype, rows, width, tokens, fp32=False):
+    """a product over random bytes: the time does not depend on the values"""
+    import torch
+    import q38hip
+    from oracle import FORMATS
+    elements, nbytes = FORMATS[qtype]
+    lib = q38hip.lib()
+    w = torch.randint(0, 120, (rows * (width // elements) * nbytes,), dtype=torch.uint8, device=device)
+    x = torch.randn(tokens, width, device=device)
+    x = x if fp32 else q38hip.quantize_q8_k(x)
+    y = torch.empty(tokens, rows, device=device)
+    tensor = q38hip.make_tensor(w.data_ptr(), qtype, width, rows, w.numel())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    entry = lib.q38hip_gemm_f32 if fp32 else lib.q38hip_gemm_q8_k
+    args = (ctypes.c_void_p(y.data_ptr()), ctypes.c_void_p(x.data_ptr()), tokens, width, ctypes.byref(tensor), stream)
+    keep = (w, x, y, tensor)
+
+    def call():
+        assert entry(*args) and keep
+    return call
+
+
+@pytest.mark.parametrize("name,rows,width,tokens,bound", (
+    ("Q3_K", 65536, 256, 1, 9.0),       # 4.4 us; 12.3 with a workgroup per eight rows
+    ("Q3_K", 65536, 256, 5, 20.0),      # 6.2; 33
+    ("IQ1_S", 65536, 256, 5, 25.0),     # 11.3; 46
+    ("IQ2_S", 248320, 256, 1, 50.0)))   # 25; 76
+def test_short_rows(device, name, rows, width, tokens, bound):
+    import oracle
+    took = best_us(product(device, getattr(oracle, name), rows, width, tokens))
+    print("%s %d x %d, %d tokens: %.1f us" % (name, rows, width, tokens, took), flush=True)
+    assert took < bound
