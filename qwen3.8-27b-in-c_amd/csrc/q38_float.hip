@@ -19,7 +19,11 @@
  * activation by a DPP row broadcast inside the fma, so a link is one
  * instruction.  Two LDS slots: at barrier k stage k + 1 is complete and the
  * last columns of stage k have been read, so its slot takes stage k + 2.  The
- * producers keep kAhead stages of loads in registers.
+ * producers keep kAhead stages of loads in registers: a quad's own header
+ * fields and quant bytes, from which its four weights are formed when the stage
+ * is stored (decoding element by element from memory at that point, a Q4_K
+ * matrix of 5120 x 5120, one token, took 320 us and one of 65536 x 768 165; 56
+ * and 25 now).
  *
  * Bound.  One token: the chain on matrices of up to 16384 rows, HBM on taller
  * ones (F32 34816 x 5120 148 us, 4.8 TB/s; F16 78 us, 4.6 TB/s).  One thread
@@ -55,28 +59,22 @@ __device__ __forceinline__ uint32_t chain_column(uint32_t c)
 }
 
 /* four consecutive chain positions of one row: what is loaded ahead, and the
- * weights it gives.  Positions past the width load nothing and give values
- * that no chain reads. */
+ * weights it gives, each the expression element_weight has.  Positions past the
+ * width load nothing and give values that no chain reads. */
 template <int T>
-struct QuadLoad {
-    template <bool Edge>
-    __device__ __forceinline__ void load(const uint8_t *, uint32_t, uint32_t) {}
-    __device__ __forceinline__ float4 weights(const uint8_t *row, uint32_t c, uint32_t width) const
-    {
-        constexpr uint32_t kElements = T == kIQ4NL ? 32 : 256;
-        float v[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t e = chain_column<T>(c + k);
-            v[k] = c + k < width ? element_weight<T>(row + (size_t)(e / kElements) * block_bytes_f(), (int)(e % kElements)) : 0.0f;
-        }
-        return make_float4(v[0], v[1], v[2], v[3]);
-    }
-    static constexpr __device__ uint32_t block_bytes_f()
-    {
-        return T == kIQ4NL ? 18 : T == kQ2K ? 84 : T == kQ3K ? 110 : T == kQ4K ? 144 : T == kQ5K ? 176 : 210;
-    }
-};
+struct QuadLoad;
+/* signed bytes of v as floats times s */
+__device__ __forceinline__ float4 scaled_bytes(float s, uint32_t v)
+{
+    return make_float4(fmul_rn(s, (float)(int8_t)v), fmul_rn(s, (float)(int8_t)(v >> 8)),
+                       fmul_rn(s, (float)(int8_t)(v >> 16)), fmul_rn(s, (float)((int32_t)v >> 24)));
+}
+/* s * q - m for the bytes q of v */
+__device__ __forceinline__ float4 scaled_minus(float s, uint32_t v, float m)
+{
+    return make_float4(__fsub_rn(fmul_rn(s, (float)(v & 255u)), m), __fsub_rn(fmul_rn(s, (float)(v >> 8 & 255u)), m),
+                       __fsub_rn(fmul_rn(s, (float)(v >> 16 & 255u)), m), __fsub_rn(fmul_rn(s, (float)(v >> 24)), m));
+}
 template <>
 struct QuadLoad<kF32> {
     float v[4];
@@ -88,7 +86,7 @@ struct QuadLoad<kF32> {
         else
             for (int k = 0; k < 4; ++k) v[k] = c + k < width ? *reinterpret_cast<const float *>(p + 4 * k) : 0.0f;
     }
-    __device__ __forceinline__ float4 weights(const uint8_t *, uint32_t, uint32_t) const
+    __device__ __forceinline__ float4 weights(uint32_t) const
     {
         return make_float4(v[0], v[1], v[2], v[3]);
     }
@@ -109,7 +107,7 @@ struct QuadLoad16 {
             v[1] = h[2] | h[3] << 16;
         }
     }
-    __device__ __forceinline__ float4 weights(const uint8_t *, uint32_t, uint32_t) const
+    __device__ __forceinline__ float4 weights(uint32_t) const
     {
         if constexpr (T == kF16)
             return make_float4(f16_to_f32(v[0]), f16_to_f32(v[0] >> 16), f16_to_f32(v[1]), f16_to_f32(v[1] >> 16));
@@ -133,11 +131,124 @@ struct QuadLoad<kQ8_0> {
             __builtin_memcpy(&q, blk + 2 + c % 32, 4);
         }
     }
-    __device__ __forceinline__ float4 weights(const uint8_t *, uint32_t, uint32_t) const
+    __device__ __forceinline__ float4 weights(uint32_t) const
     {
-        const float s = f16_to_f32(d);
-        return make_float4(fmul_rn(s, (float)(int8_t)q), fmul_rn(s, (float)(int8_t)(q >> 8)),
-                           fmul_rn(s, (float)(int8_t)(q >> 16)), fmul_rn(s, (float)((int32_t)q >> 24)));
+        return scaled_bytes(f16_to_f32(d), q);
+    }
+};
+
+/* IQ4_NL: positions 2j, 2j + 1 are elements j and 16 + j, so a quad is two bytes */
+template <>
+struct QuadLoad<kIQ4NL> {
+    uint32_t q, d;
+    template <bool Edge>
+    __device__ __forceinline__ void load(const uint8_t *row, uint32_t c, uint32_t width)
+    {
+        if (Edge) q = d = 0;
+        if (!Edge || c < width) {   /* a multiple of 32 */
+            const uint8_t *blk = row + (size_t)(c / 32) * 18;
+            d = ld16(blk);
+            q = ld16(blk + 2 + c % 32 / 2);
+        }
+    }
+    __device__ __forceinline__ float4 weights(uint32_t) const
+    {
+        return scaled_bytes(f16_to_f32(d), iq4nl_bytes((q & 15u) | (q << 4 & 0xf00u) | (q << 8 & 0xf0000u) | (q << 12 & 0xf000000u)));
+    }
+};
+/* the K-quants' widths are multiples of 256: no stage ends inside a block */
+template <>
+struct QuadLoad<kQ2K> {
+    uint32_t q, dd, sc;
+    template <bool Edge>
+    __device__ __forceinline__ void load(const uint8_t *row, uint32_t c, uint32_t)
+    {
+        const uint8_t *blk = row + (size_t)(c / 256) * 84;
+        const uint32_t i = c % 256;   /* half i / 128, field i / 32 % 4, byte i % 32 */
+        __builtin_memcpy(&q, blk + 16 + (i / 128) * 32 + i % 32, 4);
+        __builtin_memcpy(&dd, blk + 80, 4);
+        sc = blk[i / 16];
+    }
+    __device__ __forceinline__ float4 weights(uint32_t c) const
+    {
+        return scaled_minus(fmul_rn(f16_to_f32(dd), (float)(sc & 15u)), (q >> (c % 128 / 32 * 2)) & 0x03030303u,
+                            fmul_rn(f16_to_f32(dd >> 16), (float)(sc >> 4)));
+    }
+};
+template <>
+struct QuadLoad<kQ3K> {
+    uint32_t q, high, sc, sc_high, d;
+    template <bool Edge>
+    __device__ __forceinline__ void load(const uint8_t *row, uint32_t c, uint32_t)
+    {
+        const uint8_t *blk = row + (size_t)(c / 256) * 110;
+        const uint32_t i = c % 256, s = i / 16;
+        __builtin_memcpy(&q, blk + 32 + (i / 128) * 32 + i % 32, 4);
+        __builtin_memcpy(&high, blk + i % 32, 4);
+        sc = blk[96 + s % 8];
+        sc_high = blk[104 + s % 4];
+        d = ld16(blk + 108);
+    }
+    __device__ __forceinline__ float4 weights(uint32_t c) const
+    {
+        const uint32_t i = c % 256, s = i / 16;
+        const int scale = (int)((sc >> (s / 8 * 4) & 15u) | (sc_high >> (s / 4 * 2) & 3u) << 4) - 32;
+        const uint32_t absent = ~(high >> (i / 32)) & 0x01010101u;   /* minus 4 where the high bit is clear */
+        return scaled_bytes(fmul_rn(f16_to_f32(d), (float)scale),
+                            ((q >> (c % 128 / 32 * 2)) & 0x03030303u) + absent * 0xfcu);
+    }
+};
+template <int T>
+struct QuadLoadK45 {
+    uint32_t head[4], q, high;   /* d and dmin, twelve scale bytes; quants */
+    template <bool Edge>
+    __device__ __forceinline__ void load(const uint8_t *row, uint32_t c, uint32_t)
+    {
+        const uint8_t *blk = row + (size_t)(c / 256) * (T == kQ5K ? 176 : 144);
+        const uint32_t i = c % 256;
+        __builtin_memcpy(head, blk, 16);
+        __builtin_memcpy(&q, blk + (T == kQ5K ? 48 : 16) + i / 64 * 32 + i % 32, 4);
+        if (T == kQ5K) __builtin_memcpy(&high, blk + 16 + i % 32, 4);
+    }
+    __device__ __forceinline__ float4 weights(uint32_t c) const
+    {
+        const uint32_t s = c % 256 / 32, at = s % 4 * 8;
+        const uint32_t sc = s < 4 ? head[1] & 0x3f3f3f3fu : (head[3] & 0x0f0f0f0fu) | (head[1] >> 2 & 0x30303030u);
+        const uint32_t m = s < 4 ? head[2] & 0x3f3f3f3fu : (head[3] >> 4 & 0x0f0f0f0fu) | (head[2] >> 2 & 0x30303030u);
+        uint32_t v = (q >> (s % 2 * 4)) & 0x0f0f0f0fu;
+        if (T == kQ5K) v |= (high >> s & 0x01010101u) << 4;
+        return scaled_minus(fmul_rn(f16_to_f32(head[0]), (float)(sc >> at & 255u)), v,
+                            fmul_rn(f16_to_f32(head[0] >> 16), (float)(m >> at & 255u)));
+    }
+};
+template <> struct QuadLoad<kQ4K> : QuadLoadK45<kQ4K> {};
+template <> struct QuadLoad<kQ5K> : QuadLoadK45<kQ5K> {};
+/* Q6_K: positions 4j .. 4j + 3 of a half block are elements j, 32 + j, 64 + j
+ * and 96 + j: two quant bytes, one byte of their high bits, every second scale */
+template <>
+struct QuadLoad<kQ6K> {
+    uint32_t low, low32, high, sc[2], d;
+    template <bool Edge>
+    __device__ __forceinline__ void load(const uint8_t *row, uint32_t c, uint32_t)
+    {
+        const uint8_t *blk = row + (size_t)(c / 256) * 210;
+        const uint32_t half = c % 256 / 128, j = c % 128 / 4;
+        low = blk[64 * half + j];
+        low32 = blk[64 * half + 32 + j];
+        high = blk[128 + 32 * half + j];
+        __builtin_memcpy(sc, blk + 192 + 8 * half, 8);
+        d = ld16(blk + 208);
+    }
+    __device__ __forceinline__ float4 weights(uint32_t c) const
+    {
+        const uint32_t at = c % 128 / 64 * 8;   /* scales 0, 2, 4, 6 or 1, 3, 5, 7 of the half */
+        const float dv = f16_to_f32(d);
+        auto weight = [&](uint32_t nibble, int k) {
+            const int q = (int)((nibble & 15u) | (high >> (2 * k) & 3u) << 4) - 32;
+            const int s = (int8_t)(sc[k / 2] >> (16 * (k % 2) + at));
+            return fmul_rn(fmul_rn(dv, (float)s), (float)q);
+        };
+        return make_float4(weight(low, 0), weight(low32, 1), weight(low >> 4, 2), weight(low32 >> 4, 3));
     }
 };
 
@@ -215,10 +326,14 @@ struct Group {
     }
 };
 
+/* quads of five dwords and more: one stage less in registers */
+template <int T>
+constexpr bool kWideQuad = sizeof(QuadLoad<T>) > 16;
+
 /* y[t * ldy + row]: 64 rows, MT tokens in each of CW chain wavefronts, stages
  * of ST columns */
 template <int T, int MT, int CW, int ST>
-__global__ __launch_bounds__(64 * CW + kProducers, ST == 128 ? 2 : CW == 1 ? 5 : 4) void gemm_float_kernel(const uint8_t *__restrict__ w,
+__global__ __launch_bounds__(64 * CW + kProducers, ST == 128 ? 2 : CW == 1 && !kWideQuad<T> ? 5 : 4) void gemm_float_kernel(const uint8_t *__restrict__ w,
                                                                         const float *__restrict__ x,
                                                                         float *__restrict__ y, uint32_t ldy,
                                                                         uint32_t rows, uint32_t width,
@@ -226,7 +341,7 @@ __global__ __launch_bounds__(64 * CW + kProducers, ST == 128 ? 2 : CW == 1 ? 5 :
 {
     constexpr int kTok = MT * CW;
     constexpr int kFloatStage = ST, kFloatQuads = ST / 4, kGroups = ST / 16, kSlotBytes = kFloatQuads * kQuadBytes;
-    constexpr int kAhead = kTok > 16 ? 2 : 3;
+    constexpr int kAhead = kTok > 16 || kWideQuad<T> ? 2 : 3;
     constexpr int kWItems = kFloatRows * kFloatQuads / kProducers;
     constexpr int kXItems = (kTok * kFloatQuads + kProducers - 1) / kProducers;
     constexpr int kXSlot = kTok * kFloatStage * 4;
@@ -280,7 +395,7 @@ __global__ __launch_bounds__(64 * CW + kProducers, ST == 128 ? 2 : CW == 1 ? 5 :
 #pragma unroll
             for (int k = 0; k < kWItems; ++k) {
                 const int r = (tid + k * kProducers) / kFloatQuads;
-                *reinterpret_cast<float4 *>(slot + (quad / 4) * kQuadBytes + r * 16) = s.w[k].weights(wbase + wrow[k], c, width);
+                *reinterpret_cast<float4 *>(slot + (quad / 4) * kQuadBytes + r * 16) = s.w[k].weights(c);
             }
 #pragma unroll
             for (int k = 0; k < kXItems; ++k) {
@@ -385,6 +500,72 @@ __global__ __launch_bounds__(64 * CW + kProducers, ST == 128 ? 2 : CW == 1 ? 5 :
     }
 }
 
+/* One lane per row, its chain element by element: rows that fill the chip by
+ * themselves and whose weights cost more to form quad by quad than their links
+ * (row_walk says which) */
+template <int T, int MT>
+__device__ __forceinline__ void float_chain(const uint8_t *row, const float *x, uint32_t width, float *total)
+{
+    auto step = [&](float wv, uint32_t e) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) total[t] = __builtin_fmaf(wv, x[(size_t)t * width + e], total[t]);
+    };
+    if constexpr (T == kQ8_0) {
+        for (uint32_t base = 0; base < width; base += 32, row += 34) {
+            const float d = f16_to_f32(ld16(row));
+            for (int i = 0; i < 32; ++i) step(fmul_rn(d, (float)(int8_t)row[2 + i]), base + i);
+        }
+    } else if constexpr (T == kQ2K) {
+        for (uint32_t base = 0; base < width; base += 256, row += 84) {
+            const float d = f16_to_f32(ld16(row + 80)), dmin = f16_to_f32(ld16(row + 82));
+            for (int i = 0; i < 16; ++i) {
+                const float scale = fmul_rn(d, (float)(row[i] & 15)), minimum = fmul_rn(dmin, (float)(row[i] >> 4));
+                const int half = i / 8, field = (i % 8) / 2, part = i % 2;
+                for (int j = 0; j < 16; ++j) {
+                    const int q = (row[16 + 32 * half + 16 * part + j] >> (2 * field)) & 3;
+                    step(__fsub_rn(fmul_rn(scale, (float)q), minimum), base + 16 * i + j);
+                }
+            }
+        }
+    } else {
+        constexpr bool five = T == kQ5K;
+        for (uint32_t base = 0; base < width; base += 256, row += five ? 176 : 144) {
+            const float d = f16_to_f32(ld16(row)), dmin = f16_to_f32(ld16(row + 2));
+            const uint8_t *qh = row + 16, *qs = row + (five ? 48 : 16);
+            for (int c = 0; c < 4; ++c) {
+                int sc0, m0, sc1, m1;
+                k4_scale_min(2 * c, row + 4, sc0, m0);
+                k4_scale_min(2 * c + 1, row + 4, sc1, m1);
+                const float d0 = fmul_rn(d, (float)sc0), mm0 = fmul_rn(dmin, (float)m0);
+                const float d1 = fmul_rn(d, (float)sc1), mm1 = fmul_rn(dmin, (float)m1);
+                for (int i = 0; i < 32; ++i) {
+                    const int q = (qs[32 * c + i] & 15) + (five && ((qh[i] >> (2 * c)) & 1) ? 16 : 0);
+                    step(__fsub_rn(fmul_rn(d0, (float)q), mm0), base + 64 * c + i);
+                }
+                for (int i = 0; i < 32; ++i) {
+                    const int q = (qs[32 * c + i] >> 4) + (five && ((qh[i] >> (2 * c + 1)) & 1) ? 16 : 0);
+                    step(__fsub_rn(fmul_rn(d1, (float)q), mm1), base + 64 * c + 32 + i);
+                }
+            }
+        }
+    }
+}
+
+template <int T, int MT>
+__global__ __launch_bounds__(256) void gemv_float_rows(const uint8_t *__restrict__ w, const float *__restrict__ x,
+                                                       float *__restrict__ y, uint32_t ldy, uint32_t rows,
+                                                       uint32_t width, uint64_t row_bytes)
+{
+    const uint32_t row = blockIdx.x * 256u + threadIdx.x;
+    float total[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) total[t] = 0.0f;
+    float_chain<T, MT>(w + (size_t)(row < rows ? row : rows - 1) * row_bytes, x, width, total);
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+        if (row < rows) y[(size_t)t * ldy + row] = total[t];
+}
+
 template <int T, int MT, int CW, int ST = 64>
 bool launch_float(const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows, uint32_t width,
                   uint32_t row_bytes, uint32_t tokens, hipStream_t stream)
@@ -405,22 +586,52 @@ template <int T, int MT>
 bool launch_float_few(const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows, uint32_t width,
                       uint32_t row_bytes, uint32_t tokens, hipStream_t stream)
 {
-    if constexpr (T == kF32 || T == kF16 || T == kBF16 || T == kQ8_0) {
+    if constexpr (T == kF32 || T == kF16 || T == kBF16 || T == kQ8_0 || MT <= 3) {
         if ((rows + kFloatRows - 1) / kFloatRows <= 256)
             return launch_float<T, MT, 1, 128>(w, x, y, ldy, rows, width, row_bytes, tokens, stream);
     }
     return launch_float<T, MT, 1>(w, x, y, ldy, rows, width, row_bytes, tokens, stream);
 }
 
+/* Tall matrices whose rows one lane each walks: the formats and token counts
+ * (kRowTokens at most) whose element loop is the cheaper one, from 65536 rows
+ * (a wavefront per SIMD) on.  Workgroups with producers / a lane per row:
+ * Q4_K, two tokens, 65536 x 256 and 131072 x 5120 10.3 / 6.2 and 280 / 161 us,
+ * one token 131072 x 5120 278 / 246, 248320 x 1024 107 / 120; Q5_K, one token,
+ * 65536 x 5120 209 / 189, 248320 x 1024 146 / 110; 65536 x 256, one token, Q2_K
+ * 8.5 / 6.8 and Q8_0 10.2 / 8.2; 65536 x 512, two tokens, Q8_0 19 / 17.  At
+ * 49152 rows they are even or the producers win (Q4_K 49152 x 512 11.5 / 13.9).
+ * Rows of fewer than 256 columns stay with the producers, which lose there on
+ * such matrices (Q8_0 248320 x 32, four tokens 14.9 us against 5.1). */
+template <int T>
+constexpr uint32_t kRowTokens = T == kQ8_0 || T == kQ2K ? 3 : T == kQ4K ? 2 : T == kQ5K ? 1 : 0;
+template <int T>
+bool row_walk(uint32_t rows, uint32_t width, uint32_t tokens)
+{
+    if (tokens > kRowTokens<T> || rows < 65536) return false;
+    if (T == kQ5K) return true;
+    if (T == kQ4K) return tokens == 2 || width <= 256 || rows < 196608;
+    return width <= 256 || (T == kQ8_0 && width <= 512 && tokens > 1);
+}
+
 template <int T>
 bool launch_float_t(const uint8_t *w, const float *x, float *y, uint32_t ldy, uint32_t rows, uint32_t width,
                     uint32_t row_bytes, uint32_t tokens, hipStream_t stream)
 {
-    if (tokens == 1) return launch_float_few<T, 1>(w, x, y, ldy, rows, width, row_bytes, tokens, stream);
-    if constexpr (T == kF32 || T == kF16 || T == kBF16 || T == kQ8_0) {
-        if (tokens == 2) return launch_float_few<T, 2>(w, x, y, ldy, rows, width, row_bytes, tokens, stream);
-        if (tokens == 3) return launch_float_few<T, 3>(w, x, y, ldy, rows, width, row_bytes, tokens, stream);
+    if constexpr (kRowTokens<T> > 0) {
+        if (row_walk<T>(rows, width, tokens)) {
+            const dim3 grid((rows + 255) / 256), block(256);
+            if (tokens == 1) return launch_kernel(gemv_float_rows<T, 1>, grid, block, stream, w, x, y, ldy, rows, width, row_bytes);
+            if constexpr (kRowTokens<T> > 1) {
+                if (tokens == 2) return launch_kernel(gemv_float_rows<T, 2>, grid, block, stream, w, x, y, ldy, rows, width, row_bytes);
+            }
+            if constexpr (kRowTokens<T> > 2)
+                return launch_kernel(gemv_float_rows<T, 3>, grid, block, stream, w, x, y, ldy, rows, width, row_bytes);
+        }
     }
+    if (tokens == 1) return launch_float_few<T, 1>(w, x, y, ldy, rows, width, row_bytes, tokens, stream);
+    if (tokens == 2) return launch_float_few<T, 2>(w, x, y, ldy, rows, width, row_bytes, tokens, stream);
+    if (tokens == 3) return launch_float_few<T, 3>(w, x, y, ldy, rows, width, row_bytes, tokens, stream);
     if (tokens <= 4) return launch_float_few<T, 4>(w, x, y, ldy, rows, width, row_bytes, tokens, stream);
     if (tokens <= 8) return launch_float_few<T, 8>(w, x, y, ldy, rows, width, row_bytes, tokens, stream);
     /* one pass over the matrix per 32 or 64 tokens, four chain wavefronts */

@@ -39,6 +39,23 @@ def test_float_gemm_edges(device, oracle, qtype):
         run(device, oracle, qtype, rows, width, tokens, data, rng.standard_normal((tokens, width)).astype(np.float32))
 
 
+@pytest.mark.parametrize("qtype", (F32, F16, BF16, Q8_0, IQ4_NL, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K),
+                         ids=lambda t: FORMAT_NAMES[t])
+def test_float_gemm_tall(device, oracle, qtype):
+    """Above 16384 rows, where up to eight tokens take stages of 64 columns
+    (below, most take 128), and from 65536 rows on, where short rows of some
+    formats are walked by a lane each."""
+    rng = np.random.default_rng(920 + qtype)
+    elements = fc.FORMATS[qtype][0]
+    for rows, width, counts in ((16450, 67, (1, 2, 3, 4, 7)), (16385, 321, (1, 2, 3, 5)), (65601, 130, (1, 2, 3))):
+        width = -(-width // elements) * elements
+        data = fc.random_matrix(qtype, rows, width, rng)
+        x = rng.standard_normal((max(counts), width)).astype(np.float32)
+        for tokens in counts:
+            print("%s rows=%d width=%d tokens=%d" % (FORMAT_NAMES[qtype], rows, width, tokens), flush=True)
+            run(device, oracle, qtype, rows, width, tokens, data, x[:tokens])
+
+
 @pytest.mark.parametrize("qtype", (F32, F16, BF16), ids=lambda t: FORMAT_NAMES[t])
 def test_float_gemm_non_finite(device, oracle, qtype):
     rng = np.random.default_rng(950 + qtype)

@@ -1,6 +1,6 @@
 """Times of calls that once lost to the kernels they replaced.  Each bound
-lies between the two: the call takes at most two thirds of it, the form that
-was mended takes over a quarter more.  Best of several runs, GPU events."""
+lies between the two: the call takes at most two thirds of it, and the form
+that was mended takes well over it.  Best of several runs, GPU events."""
 import ctypes
 
 import pytest
@@ -47,12 +47,25 @@ def product(device, qtype, rows, width, tokens, fp32=False):
 
 
 @pytest.mark.parametrize("name,rows,width,tokens,bound", (
-    ("Q3_K", 65536, 256, 1, 9.0),       # 4.4 us; 12.3 with a workgroup per eight rows
-    ("Q3_K", 65536, 256, 5, 20.0),      # 6.2; 33
-    ("IQ1_S", 65536, 256, 5, 25.0),     # 11.3; 46
-    ("IQ2_S", 248320, 256, 1, 50.0)))   # 25; 76
+    ("Q3_K", 65536, 256, 1, 7.5),       # 4.4 us; 11 with a workgroup per eight rows
+    ("Q3_K", 65536, 256, 5, 20.0),      # 7.6; 30
+    ("IQ1_S", 65536, 256, 5, 25.0),     # 11.3; 42
+    ("IQ2_S", 248320, 256, 1, 50.0)))   # 25; 65
 def test_short_rows(device, name, rows, width, tokens, bound):
     import oracle
     took = best_us(product(device, getattr(oracle, name), rows, width, tokens))
     print("%s %d x %d, %d tokens: %.1f us" % (name, rows, width, tokens, took), flush=True)
+    assert took < bound
+
+
+@pytest.mark.parametrize("name,rows,width,tokens,bound", (
+    ("Q4_K", 96, 5120, 1, 120.0),       # 54 us; 267 with the elements of a quad decoded one by one
+    ("Q4_K", 65536, 768, 2, 50.0),      # 19; 115
+    ("Q5_K", 65536, 2048, 1, 160.0),    # 78; 325
+    ("Q2_K", 65536, 2048, 1, 110.0),    # 42; 174
+    ("IQ4_NL", 65536, 768, 1, 50.0)))   # 17; 92
+def test_float_input(device, name, rows, width, tokens, bound):
+    import oracle
+    took = best_us(product(device, getattr(oracle, name), rows, width, tokens, fp32=True), calls=20)
+    print("%s %d x %d, %d tokens, fp32 input: %.1f us" % (name, rows, width, tokens, took), flush=True)
     assert took < bound
