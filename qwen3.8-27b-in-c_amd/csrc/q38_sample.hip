@@ -20,17 +20,17 @@
  *    (float)unit * retained_total and the first candidate whose running
  *    sum exceeds it (:84-115).
  *
- * Device method.  Greedy, and more than kRankTopK candidates: each workgroup
- * selects the count best candidates of a 4096-logit chunk (count rounds of a
- * workgroup-wide best-of with the reference's order); one workgroup merges the
- * chunks' lists the same way and one thread runs the probability arithmetic
- * (expf is the C library's function restated in q38_libm.h, division correctly
- * rounded).  Up to kRankTopK candidates (every usual top_k): no rounds.  A
- * logit and its id make one 64-bit key whose order is the reference's, a set's
- * count best are found by counting how many keys of it are larger, and a first
- * count over one key per thread (per chunk) gives a bound that leaves few keys
- * for the second.  Latency bounds both forms (0.2 us of HBM): 248320 logits,
- * top_k 20: 65.8 us in rounds, 16.6 us in counts.  With a NaN
+ * Device method.  Greedy, more than kRankTopK candidates, and few candidates
+ * of a very large vocabulary (counts_select): each workgroup selects the count
+ * best candidates of a 4096-logit chunk (count rounds of a workgroup-wide
+ * best-of with the reference's order); one workgroup merges the chunks' lists
+ * the same way and one thread runs the probability arithmetic (expf is the C
+ * library's function restated in q38_libm.h, division correctly rounded).
+ * Otherwise no rounds.  A logit and its id make one 64-bit key whose order is
+ * the reference's, a set's count best are found by counting how many keys of
+ * it are larger, and a first count over one key per thread (per chunk) gives a
+ * bound that leaves few keys for the second.  Latency bounds both forms (0.2 us
+ * of HBM): 248320 logits, top_k 20: 65.8 us in rounds, 16.6 in counts.  With a NaN
  * among the adjusted logits the insertion order matters (a NaN enters the
  * last slot), so then that thread runs the reference's insertion loop
  * itself, over the whole row.
@@ -448,11 +448,21 @@ __global__ __launch_bounds__(kFinalThreads) void sample_rank_final_kernel(
 
 }  // namespace
 
+/* Whether counting selects the candidates.  Its final workgroup compares every
+ * chunk's best with every other's, so on very large vocabularies a few rounds
+ * are cheaper (rounds / counts: 2^20 logits, 2, 5 and 8 candidates 15.4 / 31.7,
+ * 23.8 / 33.1 and 33.7 / 34.1 us; 700000, 2 and 5: 15.5 / 22.4 and 23.9 / 23.6;
+ * 400000, 2: 15.3 / 15.3), as is the one round of a vocabulary of one. */
+static bool counts_select(uint32_t vocab, uint32_t count)
+{
+    return count > 1 && count <= kRankTopK && (vocab + kRankChunk - 1) / kRankChunk < 110 * count + 130;
+}
+
 size_t sample_scratch_bytes(uint32_t vocab, uint32_t top_k)
 {
     const size_t chunks = (vocab + kSampleChunk - 1) / kSampleChunk;
     const size_t count = top_k < 1 ? 1 : (top_k < vocab ? top_k : vocab);
-    if (count <= kRankTopK) {
+    if (counts_select(vocab, (uint32_t)count)) {
         const size_t rank_chunks = (vocab + kRankChunk - 1) / kRankChunk;
         return rank_chunks * count * sizeof(uint64_t) + rank_chunks * sizeof(uint32_t);
     }
@@ -478,7 +488,7 @@ bool launch_sample(uint32_t *token_out, uint64_t *state, const float *logits, ui
     const int greedy = temperature <= 0.0f || top_k <= 1;
     const uint32_t count = greedy ? 1u : (top_k < vocab ? top_k : vocab);
     const uint32_t chunks = (vocab + kSampleChunk - 1) / kSampleChunk;
-    if (!greedy && count <= kRankTopK) {
+    if (!greedy && counts_select(vocab, count)) {
         const uint32_t rank_chunks = (vocab + kRankChunk - 1) / kRankChunk;
         uint64_t *cand = static_cast<uint64_t *>(scratch);
         uint32_t *flags = reinterpret_cast<uint32_t *>(cand + (size_t)rank_chunks * count);

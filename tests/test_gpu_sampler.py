@@ -68,6 +68,17 @@ def test_selection_edges_match_reference(device, checker, top_k):
             assert device_sample(case, device) == sc.call(checker, case), case["name"]
 
 
+@pytest.mark.parametrize("vocab,top_k", ((1, 20), (358400, 2), (358401, 2), (360449, 2), (1 << 20, 2), (1 << 20, 8), (1 << 20, 9)))
+def test_large_vocabularies_match_reference(device, checker, vocab, top_k):
+    """both sides of the line between rounds (few candidates of many chunks,
+    and a vocabulary of one) and counts"""
+    rng = np.random.default_rng(vocab + top_k)
+    logits = rng.standard_normal(vocab).astype(np.float32)
+    for name, values in (("noise", logits), ("ties", np.round(logits))):
+        case = sc._case(values, rng.integers(1, 2**63), temperature=0.7, top_k=top_k, top_p=0.97, name=name)
+        assert device_sample(case, device) == sc.call(checker, case), case["name"]
+
+
 def test_state_sequence(device, checker):
     """64 consecutive draws from one row: the state carried from call to
     call as the reference carries it."""
