@@ -74,3 +74,24 @@ def test_attention_rows_bit_exact(device, oracle, context, position, rows):
     assert np.array_equal(dk.cpu().numpy()[span].view(np.uint32), kc[span].view(np.uint32))
     assert np.array_equal(np.ascontiguousarray(dv.cpu().numpy()[:, span].T).view(np.uint32), vc[span].view(np.uint32))
     assert got_q.cpu().numpy().tobytes() == oracle.quantize(want.reshape(-1)).tobytes()
+
+
+@pytest.mark.parametrize("rows", (3, 64, 90))
+def test_without_q8k_output(device, rows):
+    """The same rows without the Q8_K output, with the buffers in one small
+    allocation, in one each and in one large one."""
+    import ctypes
+    import torch
+    import q38hip
+    g = torch.Generator(device=device)
+    g.manual_seed(rows)
+    normal = lambda *shape: torch.empty(shape, device=device).normal_(0.0, 1.0, generator=g)  # noqa: E731
+    x, norm = normal(rows, 14336), 1.0 + 0.1 * normal(256)
+    keys, values = normal(rows, 1024), normal(1024, q38hip.value_pitch(rows))
+    want, _ = q38hip.attention_rows(x, norm, norm, keys, values, 0)
+    out = torch.zeros_like(want)
+    p = [ctypes.c_void_p(a) for a in (out.data_ptr(), x.data_ptr(), x.data_ptr() + 12288 * 4, x.data_ptr() + 13312 * 4,
+                                      norm.data_ptr(), keys.data_ptr(), values.data_ptr())]
+    assert q38hip.lib().q38hip_attention_rows(p[0], None, p[1], p[2], p[3], 14336, p[4], p[4], p[5], p[6], rows, 0, rows,
+                                              ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), q38hip.last_error()
+    assert torch.equal(out.view(torch.int32), want.view(torch.int32))
