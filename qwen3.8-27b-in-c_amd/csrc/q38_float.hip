@@ -326,6 +326,12 @@ struct Group {
     }
 };
 
+/* stages that hold `width` columns, up to the widest row an entry point takes */
+__host__ __device__ constexpr int stages_of(uint32_t width, uint32_t stage) { return (int)((width - 1) / stage + 1); }
+static_assert(stages_of(1, 64) == 1 && stages_of(64, 64) == 1 && stages_of(65, 64) == 2 &&
+                  stages_of(0xffffffffu, 64) == 1 << 26 && stages_of(0xffffffffu, 128) == 1 << 25,
+              "stages");
+
 /* quads of five dwords and more: one stage less in registers */
 template <int T>
 constexpr bool kWideQuad = sizeof(QuadLoad<T>) > 16;
@@ -347,7 +353,7 @@ __global__ __launch_bounds__(64 * CW + kProducers, ST == 128 ? 2 : CW == 1 && !k
     constexpr int kXSlot = kTok * kFloatStage * 4;
     __shared__ __attribute__((aligned(16))) uint8_t lds[2 * (kSlotBytes + kXSlot)];
     const uint32_t row0 = blockIdx.x * kFloatRows, tok0 = blockIdx.y * kTok;
-    const int stages = (int)((width + kFloatStage - 1) / kFloatStage);
+    const int stages = stages_of(width, kFloatStage);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 
     if (wave >= CW) {
