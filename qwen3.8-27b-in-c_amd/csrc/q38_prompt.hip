@@ -573,18 +573,39 @@ bool launch_prompt_t(const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy,
 
 }  // namespace
 
+/* The most tokens of a batch that launches of up to eight take in less time
+ * than one launch here.  A round of these workgroups takes 1.8 (Q4_K) to 2.9 us
+ * (Q6_K) per block column whatever the token count, so it loses on
+ *  - Q4_K and Q6_K matrices too small to fill the chip (launches / prompt:
+ *    1024 x 5120, 9 and 17 tokens 22 / 43 and 38 / 43 us Q4_K, 25 / 61 and 43 /
+ *    61 Q6_K; 24 tokens 82 / 39 Q4_K on 2048 rows, but 49 / 61 Q6_K on 512 and
+ *    54 / 61 on 1024; 25 tokens 55 / 61 on 512; 4096 x 5120 Q6_K 9 and 12 tokens
+ *    54 / 62 and 65 / 62; one row of 17408, 24 and 40 tokens 113 / 198 and 189 /
+ *    198 Q6_K, 25 tokens 107 / 120 Q4_K), while 34816 x 5120 at nine tokens
+ *    takes 370 / 128 and 337 / 184 us;
+ *  - short rows of tall matrices of the other formats, where the few-token
+ *    kernel walks a row with eight lanes (248320 x 256, 9 and 16 tokens IQ4_NL
+ *    48 / 112 and 69 / 115 us; 34816 x 512, 9 tokens 17 / 33).
+ * The other formats' launches are not slower than a round at 9 to about 16
+ * tokens of up to 16384 rows either (5120 x 17408, eight tokens of Q5_K 58 us
+ * against 155 for a round), which this rule leaves to the round. */
+static uint32_t few_token_limit(int type, uint32_t rows, uint32_t nb)
+{
+    if (type == kQ4K) return rows == 1 && nb > 40 ? 25 : rows < 4096 ? 23 : 8;
+    if (type == kQ6K) {
+        if (rows == 1 && nb > 40) return 40;
+        if (rows <= 1024 && nb >= 8) return nb < 20 ? 24 : rows <= 512 ? 26 : 25;
+        return rows < 4096 ? 23 : rows < 4800 ? 10 : 8;
+    }
+    return rows > 16384 && nb <= 2 ? (nb == 1 ? 16 : 12) : 8;
+}
+
 bool prompt_takes(int type, uint32_t tokens, uint32_t rows, uint32_t nb)
 {
     if (!format_takes_q8k(type) || type == kIQ1M || !rows || !nb || tokens < (uint32_t)kWideMinTokens) return false;
     /* 32-bit byte offsets inside a workgroup's rows, and the grid's limits */
     if (nb > 65536 || tokens > 65535u * 64) return false;
-    /* Q4_K and Q6_K have kernels for up to 8 tokens that beat a round of these
-     * workgroups (2.1 / 3.1 us per block column whatever the token count) on
-     * matrices too small to fill the chip: 1024 x 5120, 9 / 17 / 33 tokens 22 /
-     * 38 / 70 us in launches of 8 against 43 us (Q4_K), 25 / 43 / 79 against 61
-     * us (Q6_K).  From 4096 rows on they lose at 9 tokens already (34816 x
-     * 5120: 370 against 128 us and 337 against 184 us). */
-    return !((type == kQ4K || type == kQ6K) && rows < 4096 && tokens < 24);
+    return tokens > few_token_limit(type, rows, nb);
 }
 
 bool launch_gemm_prompt(int type, uint32_t tokens, const uint8_t *w, const uint8_t *x, float *y, uint32_t ldy,

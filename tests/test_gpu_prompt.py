@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import format_cases as fc
-from oracle import FORMAT_NAMES, IQ1_M, IQ1_S, Q2_K, Q4_K, Q5_K, Q8K_DTYPE, Q8K_FORMATS
+from oracle import FORMAT_NAMES, IQ1_M, IQ1_S, IQ4_NL, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8K_DTYPE, Q8K_FORMATS
 
 pytestmark = [pytest.mark.gpu, pytest.mark.timeout(600)]
 
@@ -81,3 +81,16 @@ def test_prompt_sums_of_one_sign_match_oracle(device, oracle, qtype):
     q8["sums"] = 32767 - rng.integers(0, 200, q8["sums"].shape)
     q8["sums"][::2] = rng.integers(0, 200, q8["sums"][::2].shape) - 32768
     check(device, oracle, qtype, rows, width, data.reshape(-1), q8, tokens)
+
+
+@pytest.mark.parametrize("qtype,rows,width,line", (
+    (Q6_K, 512, 5120, 26), (Q6_K, 1000, 2048, 24), (Q6_K, 4700, 256, 10), (Q6_K, 1, 10496, 40), (Q4_K, 1, 10496, 25),
+    (Q3_K, 16400, 256, 16), (IQ4_NL, 16390, 512, 12), (IQ1_S, 16390, 512, 12)))
+def test_either_side_of_few_token_limit(device, oracle, qtype, rows, width, line):
+    """the last batch that runs as launches of up to eight tokens, and the
+    first of one launch"""
+    rng = np.random.default_rng(880 + qtype)
+    data = fc.random_matrix(qtype, rows, width, rng)
+    q8 = oracle.quantize(rng.standard_normal((line + 1) * width).astype(np.float32))
+    for tokens in (line, line + 1):
+        check(device, oracle, qtype, rows, width, data, q8[:tokens * width // 256], tokens)

@@ -58,6 +58,18 @@ def test_short_rows(device, name, rows, width, tokens, bound):
 
 
 @pytest.mark.parametrize("name,rows,width,tokens,bound", (
+    ("Q6_K", 1, 17408, 24, 155.0),      # 113 us in launches of eight; 197 in one
+    ("Q6_K", 256, 10240, 24, 105.0),    # 90; 118
+    ("IQ4_NL", 248320, 256, 9, 75.0),   # 48; 112
+    ("Q5_K", 248320, 256, 9, 65.0)))    # 43; 91
+def test_few_tokens_of_a_batch(device, name, rows, width, tokens, bound):
+    import oracle
+    took = best_us(product(device, getattr(oracle, name), rows, width, tokens))
+    print("%s %d x %d, %d tokens: %.1f us" % (name, rows, width, tokens, took), flush=True)
+    assert took < bound
+
+
+@pytest.mark.parametrize("name,rows,width,tokens,bound", (
     ("Q4_K", 96, 5120, 1, 120.0),       # 54 us; 267 with the elements of a quad decoded one by one
     ("Q4_K", 65536, 768, 2, 50.0),      # 19; 115
     ("Q5_K", 65536, 2048, 1, 160.0),    # 78; 325
