@@ -67,3 +67,34 @@ def test_float_gemm_non_finite(device, oracle, qtype):
     x = rng.standard_normal((tokens, width)).astype(np.float32)
     x[2, 64], x[4, 130] = -np.inf, np.nan
     run(device, oracle, qtype, rows, width, tokens, data, x)
+
+
+def test_float_gemm_row_ranges(device, oracle):
+    """Rows of 64 MiB: sixty-four of them pass a workgroup's 32-bit offsets, so
+    the matrix runs in ranges of 63 rows."""
+    import torch
+    import q38hip
+    rows, width = 65, (1 << 24) + 4
+    g = torch.Generator(device=device)
+    g.manual_seed(41)
+    w = torch.empty((rows, width), device=device).normal_(0.0, 1.0, generator=g)
+    x = torch.empty((1, width), device=device).normal_(0.0, 1.0, generator=g)
+    got = q38hip.gemm_f32(w.view(torch.uint8).reshape(-1), F32, width, rows, x).cpu().numpy()[0]
+    host = x[0].cpu().numpy()
+    for row in (0, 62, 63, 64):
+        want = oracle.gemv_f32(F32, w[row].cpu().numpy().view(np.uint8), 1, host)
+        assert got[row:row + 1].view(np.uint32)[0] == np.asarray(want, np.float32).view(np.uint32)[0], row
+
+
+def test_float_gemm_token_ranges(device):
+    """More token tiles than a grid has: two launches.  Rows of one column, so
+    that an output is one product, rounded once."""
+    import torch
+    import q38hip
+    rows, tokens = 2, 65535 * 64 + 3
+    g = torch.Generator(device=device)
+    g.manual_seed(42)
+    w = torch.empty(rows, device=device).normal_(0.0, 1.0, generator=g)
+    x = torch.empty((tokens, 1), device=device).normal_(0.0, 1.0, generator=g)
+    got = q38hip.gemm_f32(w.view(torch.uint8), F32, 1, rows, x)
+    assert torch.equal(got, x * w.view(1, rows))

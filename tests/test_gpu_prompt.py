@@ -29,9 +29,10 @@ def check(device, oracle, qtype, rows, width, data, q8, tokens):
 @pytest.mark.parametrize("qtype", TYPES, ids=lambda t: FORMAT_NAMES[t])
 def test_prompt_batches_match_oracle(device, oracle, qtype):
     rng = np.random.default_rng(700 + qtype)
-    # the last shape fills the chip with 128-token workgroups
+    # at most 128 row tiles and three tiles of 64 tokens are two rounds of the
+    # chip, or one of 128-token workgroups: the last two shapes run those
     for rows, width, tokens in ((1, 256, 24), (63, 512, 64), (65, 1280, 65), (130, 5120, 33), (64, 768, 131),
-                                (4100, 256, 9), (8200, 256, 130)):
+                                (4100, 256, 9), (8200, 256, 130), (8190, 256, 130), (8130, 768, 131)):
         print("%s rows=%d width=%d tokens=%d" % (FORMAT_NAMES[qtype], rows, width, tokens), flush=True)
         data = fc.random_matrix(qtype, rows, width, rng)
         q8 = oracle.quantize(rng.standard_normal(tokens * width).astype(np.float32))
@@ -39,9 +40,10 @@ def test_prompt_batches_match_oracle(device, oracle, qtype):
 
 
 @pytest.mark.parametrize("qtype", TYPES, ids=lambda t: FORMAT_NAMES[t])
-def test_prompt_extreme_fields_match_oracle(device, oracle, qtype):
+@pytest.mark.parametrize("rows,tokens", ((40, 26), (8150, 129)))
+def test_prompt_extreme_fields_match_oracle(device, oracle, qtype, rows, tokens):
     rng = np.random.default_rng(800 + qtype)
-    rows, width, tokens = 40, 512, 26
+    width = 512
     data = fc.random_matrix(qtype, rows, width, rng).reshape(rows, -1)
     scales = fc.random_matrix(qtype, rows, width, rng).reshape(rows, -1)
     data[:20][data[:20] < 128] = 0      # rows of 0x00 and 0xff bytes
