@@ -326,8 +326,11 @@ struct Group {
     }
 };
 
-/* stages that hold `width` columns, up to the widest row an entry point takes */
-__host__ __device__ constexpr int stages_of(uint32_t width, uint32_t stage) { return (int)((width - 1) / stage + 1); }
+/* stages that hold `width` columns, up to the widest row an entry point takes.
+ * The host passes the count: worked out in the kernel this way, the compiler
+ * orders the producers' loads differently and eight tokens take longer (F16
+ * 5120 x 6144 121 against 104 us). */
+constexpr int stages_of(uint32_t width, uint32_t stage) { return (int)((width - 1) / stage + 1); }
 static_assert(stages_of(1, 64) == 1 && stages_of(64, 64) == 1 && stages_of(65, 64) == 2 &&
                   stages_of(0xffffffffu, 64) == 1 << 26 && stages_of(0xffffffffu, 128) == 1 << 25,
               "stages");
@@ -343,7 +346,7 @@ __global__ __launch_bounds__(64 * CW + kProducers, ST == 128 ? 2 : CW == 1 && !k
                                                                         const float *__restrict__ x,
                                                                         float *__restrict__ y, uint32_t ldy,
                                                                         uint32_t rows, uint32_t width,
-                                                                        uint32_t row_bytes, uint32_t tokens)
+                                                                        uint32_t row_bytes, uint32_t tokens, int stages)
 {
     constexpr int kTok = MT * CW;
     constexpr int kFloatStage = ST, kFloatQuads = ST / 4, kGroups = ST / 16, kSlotBytes = kFloatQuads * kQuadBytes;
@@ -353,7 +356,6 @@ __global__ __launch_bounds__(64 * CW + kProducers, ST == 128 ? 2 : CW == 1 && !k
     constexpr int kXSlot = kTok * kFloatStage * 4;
     __shared__ __attribute__((aligned(16))) uint8_t lds[2 * (kSlotBytes + kXSlot)];
     const uint32_t row0 = blockIdx.x * kFloatRows, tok0 = blockIdx.y * kTok;
-    const int stages = stages_of(width, kFloatStage);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 
     if (wave >= CW) {
@@ -578,7 +580,8 @@ bool launch_float(const uint8_t *w, const float *x, float *y, uint32_t ldy, uint
 {
     return launch_kernel(gemm_float_kernel<T, MT, CW, ST>,
                          dim3((rows + kFloatRows - 1) / kFloatRows, (tokens + MT * CW - 1) / (MT * CW)),
-                         dim3(64 * CW + kProducers), stream, w, x, y, ldy, rows, width, row_bytes, tokens);
+                         dim3(64 * CW + kProducers), stream, w, x, y, ldy, rows, width, row_bytes, tokens,
+                         stages_of(width, ST));
 }
 
 /* Up to eight tokens.  The types of real float matrices (GGUF files keep
