@@ -234,15 +234,15 @@ __device__ __forceinline__ void decode_walk(const uint8_t *blk, int l, const uin
  * 4.4 and 32.9 / 8.0 us, IQ1_S 17.2 / 7.7 and 45.4 / 11.3; 8192 x 768, five
  * tokens, Q3_K 6.4 / 5.7), up to as many blocks as where the codebook in LDS
  * or, from four tokens on, the shared activations win again (65536 x 1536 and
- * 65536 x 5120, one token, IQ2_S 41 / 39 and 96 / 127 us; 65536 x 5120 Q3_K 54 /
- * 48; 65536 x 2048 and 65536 x 3072, five tokens, IQ2_S 78 / 73 and 98 / 108).
+ * 65536 x 5120, one token, IQ2_S 41 / 39 and 96 / 127 us; 65536 x 1280 IQ1_S 27 /
+ * 32, IQ2_S 36 / 33; 65536 x 5120 Q3_K 54 / 48; 65536 x 2048 and 65536 x 3072, five tokens, IQ2_S 78 / 73 and 98 / 108).
  * An IQ1_S walk is still 3 to 9 % behind the kernel that stood here before the
  * block ranges (65536 x 256, five tokens 10.5 us). */
 template <int T, int MT>
 bool walk_rows(uint32_t rows, uint32_t nb)
 {
-    constexpr bool book = table_dwords<T>() > 0;
-    const uint32_t most = book ? (MT > 3 ? 6 : 4) + (rows >= 65536 ? 2 : 0) : MT > 3 ? 10 : 20;
+    constexpr bool book = table_dwords<T>() > 0, gains = MT > 3 || T == kIQ2S || T == kIQ2XS;
+    const uint32_t most = book ? (MT > 3 ? 6 : 4) + (gains && rows >= 65536 ? 2 : 0) : MT > 3 ? 10 : 20;
     return T == kIQ4NL || (nb <= most && rows >= 2700 * nb);
 }
 
@@ -254,7 +254,7 @@ void gemv_rows_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__
                       uint32_t rows, uint32_t nb, const uint32_t *__restrict__ iq1s_grid)
 {
     const int l = threadIdx.x & 7;
-    const uint32_t row = blockIdx.x * 32u + (threadIdx.x >> 3);
+    const uint32_t row = (blockIdx.x * 256u + threadIdx.x) >> 3;
     const uint8_t *wr = w + (size_t)(row < rows ? row : rows - 1) * nb * block_bytes<T>();
     const uint32_t *table = table_of<T>(iq1s_grid);
     float acc[MT], scalar[MT];
@@ -324,8 +324,14 @@ void launch_format_typed(const uint8_t *w, const uint8_t *x, float *y, uint32_t 
             return;
         }
     }
-    hipLaunchKernelGGL((gemv_rows_kernel<T, MT>), dim3((rows + 31) / 32), dim3(256), 0, stream, w, x, y, ldy, rows, nb,
-                       iq1s);
+    /* eight lanes per row in 32-bit thread numbers */
+    constexpr uint32_t kRange = 1u << 28;
+    for (uint32_t r = 0; r < rows; r += kRange) {
+        const uint32_t n = rows - r < kRange ? rows - r : kRange;
+        hipLaunchKernelGGL((gemv_rows_kernel<T, MT>), dim3((n + 31) / 32), dim3(256), 0, stream,
+                           w + (size_t)r * nb * block_bytes<T>(), x, y + r, ldy, n, nb, iq1s);
+        if (rows - r <= kRange) break;
+    }
 }
 
 template <int T>
