@@ -171,9 +171,10 @@ __global__ __launch_bounds__(64 * H) void gemv_format_kernel(const uint8_t *__re
 /* decode_lane for gemv_rows_kernel: with few blocks to a row, formats with
  * several header fields per group are faster loading the bytes a lane uses than
  * whole headers to shift them from (65536 x 1024, one token: IQ2_S 27 against
- * 32 us, IQ1_S 26 against 28 us) */
+ * 32 us, IQ1_S 26 against 28 us).  m (IQ1_S): the factor of activation sums 2l
+ * and 2l + 1, from the header of group l that the lane has anyway. */
 template <int T>
-__device__ __forceinline__ void decode_walk(const uint8_t *blk, int l, const uint32_t *table, LaneBlock &b)
+__device__ __forceinline__ void decode_walk(const uint8_t *blk, int l, const uint32_t *table, LaneBlock &b, int &m)
 {
     const int sec = l >> 1, half = l & 1;
     if constexpr (T == kIQ2S) {
@@ -199,6 +200,7 @@ __device__ __forceinline__ void decode_walk(const uint8_t *blk, int l, const uin
             const uint32_t index = blk[2 + 4 * g + sec] | (((high >> (3 * sec)) & 7u) << 8);
             b.q[g] = table[2 * index + half];
             b.s[g] = 1 + 2 * (int)((high >> 12) & 7u);
+            if (l == g) m = high & 0x8000u ? -b.s[g] : b.s[g];
         }
         b.d = f16_to_f32(ld16(blk));
     } else if constexpr (T == kQ3K) {
@@ -238,8 +240,8 @@ __device__ __forceinline__ void decode_walk(const uint8_t *blk, int l, const uin
  * or, from four tokens on, the shared activations win again (65536 x 1536 and
  * 65536 x 5120, one token, IQ2_S 41 / 39 and 96 / 127 us; 65536 x 1280 IQ1_S 27 /
  * 32, IQ2_S 36 / 33; 65536 x 5120 Q3_K 54 / 48; 65536 x 2048 and 65536 x 3072, five tokens, IQ2_S 78 / 73 and 98 / 108).
- * An IQ1_S walk is still 3 to 9 % behind the kernel that stood here before the
- * block ranges (65536 x 256, five tokens 10.5 us). */
+ * An IQ1_S walk of four to seven tokens is still 2 to 5 % behind the kernel
+ * that stood here before the block ranges (65536 x 2048, five tokens 67 / 70). */
 template <int T, int MT>
 bool walk_rows(uint32_t rows, uint32_t nb)
 {
@@ -265,9 +267,10 @@ void gemv_rows_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__
     for (uint32_t b = 0; b < nb; ++b) {
         const uint8_t *blk = wr + (size_t)b * block_bytes<T>();
         LaneBlock lb;
-        decode_walk<T>(blk, l, table, lb);
         int m0 = 0, m1 = 0;
-        if constexpr (has_extra<T>()) extra_factors<T>(blk, l, m0, m1);
+        decode_walk<T>(blk, l, table, lb, m0);
+        if constexpr (T == kIQ1S) m1 = m0;
+        else if constexpr (has_extra<T>()) extra_factors<T>(blk, l, m0, m1);
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             const uint8_t *xb = x + ((size_t)t * nb + b) * kQ8KBytes;
